@@ -780,6 +780,7 @@ struct KernelArgs {
         int ehs_batch;
         uint32_t tail_del_lanes; /* resident lanes of the stepping launch */
         int lanes_per_wave;      /* lanes of a wavefront taking histories */
+        int lanes_auto;          /* fewer in the rounds that fit (k_step) */
         int tail_adaptive;       /* in-wavefront DELs chosen per round */
         Recorder rec;
         unsigned long long * counters;
@@ -1040,10 +1041,6 @@ __global__ void __launch_bounds__(512, 2) k_step(KernelArgs args, int parity)
         const EngineT<F32, FT, ST> eng = { a.p, a.mv, a.c, a.g, *ft, *st,
                 a.rec };
         const uint64_t below = lanes_below();
-        /* Lanes of the wavefront that take histories: all of them, or the
-         * first lanes_per_wave when a small batch is spread over the
-         * device. */
-        const bool lane_on = (int)(threadIdx.x & 63) < a.lanes_per_wave;
         const uint32_t * in = a.q_step[parity];
         const unsigned long long n_in = a.counters[C_STEP_N0 + parity];
         if (n_in == 0) return;
@@ -1071,6 +1068,33 @@ __global__ void __launch_bounds__(512, 2) k_step(KernelArgs args, int parity)
         w.phase = PHASE_EMPTY;
         uint32_t slot = 0;
         bool exhausted = false;
+        /* Lanes of the wavefront that take histories. */
+        int lanes = a.lanes_per_wave;
+        if (n_in <= a.tail_del_lanes) {
+                /* The round fits in the resident lanes: each wavefront takes
+                 * its share of the queue once, and the queue has nothing
+                 * more for it. (Taken from the shared counter instead, a
+                 * wavefront learns that only when it asks again, with a
+                 * lane freed by its first DEL: with one history per
+                 * wavefront every DEL cost a round.) The shares are spread
+                 * over all wavefronts, first over the blocks, then over the
+                 * wavefronts of a block, unless the caller asked for a
+                 * number of lanes. */
+                const uint32_t waves =
+                    gridDim.x * (blockDim.x >> 6);
+                if (a.lanes_auto)
+                        lanes = (int)((n_in + waves - 1) / waves);
+                const uint32_t wave =
+                    (threadIdx.x >> 6) * gridDim.x + blockIdx.x;
+                const unsigned long long k =
+                    (unsigned long long)wave * lanes + (threadIdx.x & 63);
+                if (((int)(threadIdx.x & 63) < lanes) && (k < n_in)) {
+                        slot = in[k];
+                        w = a.records[slot];
+                }
+                exhausted = true;
+        }
+        const bool lane_on = (int)(threadIdx.x & 63) < lanes;
         unsigned long long steps_acc = 0;
         for (;;) {
                 /* Hand over the histories that left the stepping phase. */
@@ -1319,15 +1343,12 @@ enum pumas_return transport_chunk(const KernelArgs & a0, size_t base,
          * the rest of the device to concurrent requests. */
         const size_t resident = (size_t)L.n_cu * L.per_cu;
         const size_t waves = (size_t)(L.block / 64);
-        int lanes = L.lanes_per_wave;
-        if (lanes <= 0) {
-                /* Spread: as many histories per wavefront as it takes for
-                 * the batch to fill every resident wavefront. */
-                const size_t per = (m + resident * waves - 1) /
-                    (resident * waves);
-                lanes = (per < 1) ? 1 : (per > 64 ? 64 : (int)per);
-        }
-        const size_t per_block = waves * (size_t)lanes;
+        /* Spread (0): as many blocks as histories, up to all the resident
+         * ones; a round that fits in them shares its histories out over
+         * every wavefront (k_step). */
+        const bool lanes_auto = L.lanes_per_wave <= 0;
+        const int lanes = lanes_auto ? 64 : L.lanes_per_wave;
+        const size_t per_block = lanes_auto ? 1 : waves * (size_t)lanes;
         const size_t fill = (m + per_block - 1) / per_block;
         L.step_grid = (unsigned)((fill < resident) ? (fill > 0 ? fill : 1) :
                                                      resident);
@@ -1339,6 +1360,7 @@ enum pumas_return transport_chunk(const KernelArgs & a0, size_t base,
         hipStream_t stream = L.stream;
         KernelArgs a = a0;
         a.lanes_per_wave = lanes;
+        a.lanes_auto = lanes_auto;
         a.tail_del_lanes = L.step_grid * (uint32_t)(waves * lanes);
         a.tail_adaptive = (L.tail_del == 0);
         a.states = a0.states + base;

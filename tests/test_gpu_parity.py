@@ -276,3 +276,21 @@ def test_lanes_per_wave_invariance(gpu_standard, lanes):
     assert (alt.states == ref.states).all()
     for k in ("events", "media", "steps", "draws", "rc"):
         np.testing.assert_array_equal(getattr(alt, k), getattr(ref, k))
+
+
+@pytest.mark.parametrize("n", [1, 255, 257, 16383, 16384, 16385, 33001])
+def test_round_sizes_invariance(gpu_standard, n):
+    """A round that fits in the resident lanes (here 256 CUs x one wavefront
+    = 16384) shares its histories out over the wavefronts; a larger one
+    hands them out from a counter. Both, and the rounds without discrete
+    losses in the wavefronts, give the same results."""
+    s = W.slabs_forward_states(n, seed=18)
+    geom = pa.Geometry(gpu_standard, W.slabs_geometry())
+    ctx = W.slabs_forward_context()
+    ref = pa.transport(gpu_standard, ctx, geom, s.copy(), seed=18,
+                       lanes_per_wave=64, tail_del=-1)
+    alt = pa.transport(gpu_standard, ctx, geom, s.copy(), seed=18,
+                       block_size=64, blocks_per_cu=1)
+    assert (alt.states == ref.states).all()
+    for k in ("events", "media", "steps", "draws", "rc"):
+        np.testing.assert_array_equal(getattr(alt, k), getattr(ref, k))
