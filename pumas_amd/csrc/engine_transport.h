@@ -57,7 +57,9 @@ struct Walker {
          * step_max_locals: the locals step times the accuracy (0: uniform
          * medium). */
         double density, step_max_medium, step_max_locals;
-        double ti, wi, Xi, Xf, dei, grammage_max;
+        double ti, wi, dei, grammage_max;
+        /* Index of the history's record (lean engines only). */
+        uint32_t slot;
 };
 
 /* A recorded frame: layout of struct pumas_gpu_frame (include/pumas_gpu.h),
@@ -150,6 +152,9 @@ static PG_NOINLINE void record_state(const Recorder rec, const Track t,
         f.reserved = 0;
 }
 
+/* SCHEME of an engine that reads the energy loss mode from its Config. */
+constexpr int SCHEME_ANY = -2;
+
 /*
  * The transport engine. With F32 false every operation is the reference's
  * FP64 arithmetic. With F32 true (FP32-bulk) the per-step table lookups,
@@ -158,7 +163,8 @@ static PG_NOINLINE void record_state(const Recorder rec, const Track t,
  * direction), the range to energy inversion, the event weights and the
  * geometry stay in double precision.
  */
-template <bool F32, class FT = FloatTables, class ST = PhysicsView>
+template <bool F32, class FT = FloatTables, class ST = PhysicsView,
+    bool LEAN = false, int SCHEME = SCHEME_ANY>
 struct EngineT {
         const PhysicsView & p;
         const ModelView & mv;
@@ -169,13 +175,37 @@ struct EngineT {
          * copy of them in LDS). */
         const ST & st;
         Recorder rec;
+        /* LEAN: the records of the histories in flight. */
+        Walker * records = nullptr;
+
+        /* The members of a Walker that only its events and its end touch
+         * (ids and end conditions, the limits of the other energy loss
+         * modes): a lean engine, which keeps the rest of the Walker in
+         * registers over many steps, leaves them in the record. A lean
+         * engine does not record frames. */
+        PG_FN Walker & cold(Walker & w) const
+        {
+                if constexpr (LEAN)
+                        return records[w.slot];
+                else
+                        return w;
+        }
 
         /* Records the state of `w` in `medium` with `event`, if the history
          * is recorded (record_state, src/pumas.c:7738-7780). */
         PG_FN void record_frame(const Walker & w, int medium, int event) const
         {
-                if (!w.record) return;
-                record_state(rec, w.t, medium, event);
+                if constexpr (!LEAN) {
+                        if (!w.record) return;
+                        record_state(rec, w.t, medium, event);
+                }
+        }
+
+        /* The energy loss mode (a constant when the engine is compiled for
+         * one). */
+        PG_FN int loss() const
+        {
+                return (SCHEME == SCHEME_ANY) ? c.energy_loss : SCHEME;
         }
 
         /* Per-step table lookups, in the bulk precision. */
@@ -316,7 +346,7 @@ struct EngineT {
                 const double r = sqrt(-2. * lm::log(t.rng.uniform()));
                 const double phi = 2. * PI * t.rng.uniform();
                 double s, cp;
-                lm::sincos(phi, &s, &cp);
+                lm::sincos_near(phi, &s, &cp);
                 t.randn_next = r * cp;
                 return r * s;
         }
@@ -364,7 +394,7 @@ struct EngineT {
                         sp = sf;
                 } else {
                         const double phi = PI * (1. - 2. * t.rng.uniform());
-                        lm::sincos(phi, &sp, &cp);
+                        lm::sincos_near(phi, &sp, &cp);
                 }
                 direction[0] =
                     cos_theta * direction[0] + st * (cp * u0x + sp * u1x);
@@ -614,7 +644,7 @@ struct EngineT {
                         *grammage_max = 0.;
                 }
 
-                const int scheme = c.energy_loss;
+                const int scheme = loss();
                 if (scheme == MODE_DISABLED) {
                         if (c.scattering == MODE_MIXED) {
                                 const double X = Xi -
@@ -687,7 +717,7 @@ struct EngineT {
         PG_FN void step_fluctuate(Track & t, int material, double Xtot,
             double dX, double * kf, double * ratio) const
         {
-                const int scheme = c.energy_loss;
+                const int scheme = loss();
                 const double s = sgn();
                 double k1, r = 0.;
                 k1 = cel_kinetic_energy(st, t.ix, scheme, material, Xtot - s * dX);
@@ -744,14 +774,15 @@ struct EngineT {
         /* step_transport, src/pumas.c:6296-6925 (no magnetic field).
          * `density_io` holds the local density at the start of the step and
          * receives the one at its end; `step_max_locals` the locals step,
-         * updated at the end of the step. Returns the end medium through
+         * updated at the end of the step. `ct` holds the cold members (`t`
+         * itself, but for lean engines). Returns the end medium through
          * `out_medium`. */
-        PG_FN void step_transport(Track & t, int straight, int medium,
+        PG_FN void step_transport(Track & t, Track & ct, int straight, int medium,
             int material, double & density_io, double & step_max_locals,
             double grammage_max, double step_max_medium, int step_max_type,
             int * out_medium) const
         {
-                const int scheme = c.energy_loss;
+                const int scheme = loss();
                 double * const direction = t.dir;
                 double * const position = t.pos;
                 const double density = density_io;
@@ -900,25 +931,28 @@ struct EngineT {
                 const double dX = 0.5 * step * (density + locals_density);
                 if ((scheme >= MODE_CSDA) && (scheme <= MODE_MIXED)) {
                         const double X = Xtot - sg * dX;
+                        const double X_limit = (c.event & EVENT_LIMIT_ENERGY) ?
+                            ct.step_X_limit :
+                            0.;
                         if ((c.direction == MODE_FORWARD) &&
-                            (X <= t.step_X_limit)) {
+                            (X <= X_limit)) {
                                 k1 = (c.event & EVENT_LIMIT_ENERGY) ?
                                     c.limit_energy :
                                     0.;
                                 const double grammage =
-                                    t.grammage + Xtot - t.step_X_limit;
+                                    t.grammage + Xtot - X_limit;
                                 if ((grammage_max <= 0.) ||
                                     (grammage < grammage_max)) {
                                         grammage_max = grammage;
                                         event = EVENT_LIMIT_ENERGY;
                                 }
                         } else if ((c.direction == MODE_BACKWARD) &&
-                            (t.step_X_limit > 0.) && (X > t.step_X_limit)) {
+                            (X_limit > 0.) && (X > X_limit)) {
                                 k1 = (c.event & EVENT_LIMIT_ENERGY) ?
                                     c.limit_energy :
                                     0.;
                                 const double grammage =
-                                    t.grammage + t.step_X_limit - Xtot;
+                                    t.grammage + X_limit - Xtot;
                                 if ((grammage_max <= 0.) ||
                                     (grammage < grammage_max)) {
                                         grammage_max = grammage;
@@ -1084,8 +1118,8 @@ struct EngineT {
                 double time_max =
                     (c.event & EVENT_LIMIT_TIME) ? c.limit_time : 0.;
                 if (c.decay == MODE_RANDOMISED) {
-                        if ((time_max <= 0.) || (t.lifetime < time_max)) {
-                                time_max = t.lifetime;
+                        if ((time_max <= 0.) || (ct.lifetime < time_max)) {
+                                time_max = ct.lifetime;
                                 decayed = 1;
                         }
                 }
@@ -1103,7 +1137,7 @@ struct EngineT {
                                         if (Xi + dxT < t.grammage) {
                                                 event = EVENT_LIMIT_TIME;
                                                 t.time = time_max;
-                                                t.decayed = decayed;
+                                                ct.decayed = decayed;
                                                 step = dxT * density_i;
                                                 if (step > sf1) step = sf1;
                                                 t.grammage = Xi + dxT;
@@ -1128,7 +1162,7 @@ struct EngineT {
                         if ((time_max > 0.) && (t.time >= time_max)) {
                                 event = EVENT_LIMIT_TIME;
                                 t.time = time_max;
-                                t.decayed = decayed;
+                                ct.decayed = decayed;
 
                                 const double a = (momentum / p_f - 1.) / sf1;
                                 const double cc =
@@ -1714,12 +1748,12 @@ struct EngineT {
                  * mode; FP32-bulk reads its single precision mirrors. */
                 if constexpr (F32) {
                         float m, l;
-                        ftable_get_msc(ft, t.fx, c.energy_loss, material,
+                        ftable_get_msc(ft, t.fx, loss(), material,
                             (float)kinetic, &m, &l);
                         mu0 = m;
                         invlb1 = l;
                 } else
-                        table_get_msc(st, t.ix, c.energy_loss, material,
+                        table_get_msc(st, t.ix, loss(), material,
                             kinetic, &mu0, &invlb1);
 
                 const int nc = p.elements_in[material];
@@ -1887,13 +1921,13 @@ struct EngineT {
 
                 int do_stepping = 1;
                 if ((step_max_medium <= 0.) && (step_max_locals <= 0.) &&
-                    (c.energy_loss <= MODE_CSDA)) {
-                        if ((c.energy_loss == MODE_DISABLED) &&
+                    (loss() <= MODE_CSDA)) {
+                        if ((loss() == MODE_DISABLED) &&
                             ((c.event & EVENT_LIMIT) == 0)) {
                                 w.rc = RETURN_MISSING_LIMIT;
                                 return;
                         } else if ((c.scattering == MODE_DISABLED) &&
-                            (c.energy_loss == MODE_CSDA)) {
+                            (loss() == MODE_CSDA)) {
                                 do_stepping = 0;
                         }
                 }
@@ -1919,7 +1953,7 @@ struct EngineT {
                 w.step_max_medium = step_max_medium;
                 w.step_max_locals = step_max_locals;
                 w.step_max_type = step_max_type;
-                const int scheme = c.energy_loss;
+                const int scheme = loss();
                 w.straight = ((c.scattering == MODE_DISABLED) &&
                                  (scheme <= MODE_MIXED) &&
                                  (step_max_locals <= 0.)) ?
@@ -1928,14 +1962,13 @@ struct EngineT {
                 t.step_event = EVENT_NONE;
                 w.ti = t.time;
                 w.wi = t.weight;
-                w.Xi = t.grammage;
+                double Xf = 0.;
+                w.dei = 0.;
                 if (scheme > MODE_DISABLED) {
                         const double ki = t.energy;
-                        w.Xf = cel_grammage(p, t.ix, scheme, material, ki);
+                        Xf = cel_grammage(p, t.ix, scheme, material, ki);
                         w.dei = 1. /
                             cel_energy_loss(p, t.ix, scheme, material, ki);
-                } else {
-                        w.Xf = w.dei = 0.;
                 }
 
                 if ((c.event & EVENT_LIMIT_DISTANCE) &&
@@ -1967,7 +2000,7 @@ struct EngineT {
                         material, c.limit_energy) :
                     0.;
                 t.step_invlb1 = 0;
-                transport_limit(t, material, w.Xi, w.Xf, &w.grammage_max);
+                transport_limit(t, material, t.grammage, Xf, &w.grammage_max);
                 if (t.step_event) {
                         w.event = t.step_event;
                         return;
@@ -1980,6 +2013,7 @@ struct EngineT {
         PG_FN void walker_finish(Walker & w) const
         {
                 Track & t = w.t;
+                Walker & cw = cold(w);
                 if (c.direction == MODE_FORWARD) {
                         const double kinetic_min =
                             (c.event & EVENT_LIMIT_ENERGY) ? c.limit_energy :
@@ -1991,11 +2025,11 @@ struct EngineT {
                             (fabs(t.energy - c.limit_energy) < FLT_EPS))
                                 t.energy = c.limit_energy;
                 }
-                w.end_medium = w.medium;
-                w.event = t.step_event;
+                cw.end_medium = w.medium;
+                cw.event = t.step_event;
                 w.phase = PHASE_DONE;
-                if ((t.max_steps < 0) && (w.rc == RETURN_SUCCESS))
-                        w.rc = (t.max_steps == MARK_LOOP_LIMIT) ?
+                if ((t.max_steps < 0) && (cw.rc == RETURN_SUCCESS))
+                        cw.rc = (t.max_steps == MARK_LOOP_LIMIT) ?
                             HISTORY_LOOP_LIMIT :
                             HISTORY_NO_TARGET;
                 record_frame(w, w.medium, t.step_event | EVENT_STOP);
@@ -2006,17 +2040,23 @@ struct EngineT {
         PG_FN void walker_post(Walker & w) const
         {
                 Track & t = w.t;
-                const int scheme = c.energy_loss;
+                const int scheme = loss();
                 w.ti = t.time;
-                w.wi = t.weight;
-                w.Xi = t.grammage;
-                if (c.energy_loss >= MODE_CSDA) {
-                        const double ki = t.energy;
-                        w.Xf = cel_grammage(p, t.ix, scheme, w.material, ki);
+                /* A lean engine's weight changes at events only, each of
+                 * which ends here: its initial weight is the weight. */
+                if constexpr (!LEAN) w.wi = t.weight;
+                /* The grammage is read by the limits of the CSDA and mixed
+                 * modes only, the energy loss by the backward weights. */
+                const double Xi = t.grammage;
+                double Xf = 0.;
+                if ((scheme >= MODE_CSDA) && (scheme <= MODE_MIXED))
+                        Xf = cel_grammage(
+                            p, t.ix, scheme, w.material, t.energy);
+                if ((scheme >= MODE_CSDA) && (c.direction == MODE_BACKWARD))
                         w.dei = 1. /
-                            cel_energy_loss(p, t.ix, scheme, w.material, ki);
-                }
-                transport_limit(t, w.material, w.Xi, w.Xf, &w.grammage_max);
+                            cel_energy_loss(
+                                p, t.ix, scheme, w.material, t.energy);
+                transport_limit(t, w.material, Xi, Xf, &w.grammage_max);
                 if (t.step_event)
                         walker_finish(w);
                 else
@@ -2028,7 +2068,7 @@ struct EngineT {
         PG_FN void walker_step(Walker & w) const
         {
                 Track & t = w.t;
-                const int scheme = c.energy_loss;
+                const int scheme = loss();
                 if (w.step_index > 1) {
                         int unused;
                         w.step_max_type =
@@ -2046,7 +2086,7 @@ struct EngineT {
                          * the cap below, as in the reference, which has no
                          * end for it: the history ends at once with a value
                          * error. */
-                        w.rc = RETURN_VALUE_ERROR;
+                        cold(w).rc = RETURN_VALUE_ERROR;
                         t.step_event = EVENT_LIMIT;
                         walker_finish(w);
                         return;
@@ -2055,33 +2095,36 @@ struct EngineT {
                         /* The step cap, or a history marked by a loop that
                          * gave up or by a failed target selection: it ends
                          * here with no event and a status code. */
-                        if (t.max_steps >= 0) w.rc = HISTORY_STEP_LIMIT;
+                        if (t.max_steps >= 0) cold(w).rc = HISTORY_STEP_LIMIT;
                         t.step_event = EVENT_NONE;
                         walker_finish(w);
                         return;
                 }
 
                 int new_medium = -1;
-                step_transport(t, w.straight, w.medium, w.material, w.density,
+                const int straight =
+                    (SCHEME == MODE_STRAGGLED) ? 0 : w.straight;
+                step_transport(t, cold(w).t, straight, w.medium, w.material, w.density,
                     w.step_max_locals, w.grammage_max, w.step_max_medium,
                     w.step_max_type, &new_medium);
                 w.step_index++;
                 /* Recorded steps, src/pumas.c:5296-5328: every period-th
                  * step also gets the event-time weight update. */
-                const int record_step = w.record && (rec.period > 0) &&
+                const int record_step = !LEAN && w.record && (rec.period > 0) &&
                     (w.step_index != 1) && ((w.step_index % rec.period) == 0);
                 if (!t.step_event && !record_step) return;
 
                 if ((c.direction == MODE_BACKWARD) &&
-                    (c.energy_loss >= MODE_CSDA)) {
+                    (loss() >= MODE_CSDA)) {
                         const double wt = (c.decay == MODE_WEIGHTED) ?
                             lm::exp(-fabs(t.time - w.ti) / p.ctau) :
                             1.;
-                        t.weight = w.wi * wt * w.dei *
+                        t.weight = (LEAN ? t.weight : w.wi) * wt * w.dei *
                             cel_energy_loss(p, t.ix, scheme, w.material,
                                 t.energy);
                 } else if (c.decay == MODE_WEIGHTED) {
-                        t.weight = w.wi * lm::exp(-fabs(t.time - w.ti) / p.ctau);
+                        t.weight = (LEAN ? t.weight : w.wi) *
+                            lm::exp(-fabs(t.time - w.ti) / p.ctau);
                 }
 
                 if (!t.step_event) {
@@ -2106,12 +2149,16 @@ struct EngineT {
                                          (w.step_max_locals <= 0.)) ?
                             1 :
                             0;
-                        const int tmp_scheme =
-                            scheme > MODE_DISABLED ? scheme : MODE_CSDA;
-                        t.step_X_limit = (c.event & EVENT_LIMIT_ENERGY) ?
-                            cel_grammage(p, t.ix, tmp_scheme, w.material,
-                                c.limit_energy) :
-                            0.;
+                        /* Read in the CSDA and mixed modes only. */
+                        if (scheme < MODE_STRAGGLED) {
+                                const int tmp_scheme =
+                                    scheme > MODE_DISABLED ? scheme : MODE_CSDA;
+                                cold(w).t.step_X_limit =
+                                    (c.event & EVENT_LIMIT_ENERGY) ?
+                                    cel_grammage(p, t.ix, tmp_scheme,
+                                        w.material, c.limit_energy) :
+                                    0.;
+                        }
                         t.step_first = 1;
                         t.step_invlb1 = 0;
                         if (!(c.event & EVENT_MEDIUM))
@@ -2129,6 +2176,17 @@ struct EngineT {
                             w.t, w.medium, &w.material, &w.density);
         }
 
+        static PG_FN void del_members(Track & to, const Track & from)
+        {
+                to.energy = from.energy;
+                to.weight = from.weight;
+                for (int i = 0; i < 3; i++) to.dir[i] = from.dir[i];
+                to.step_event = from.step_event;
+                to.max_steps = from.max_steps;
+                to.ix = from.ix;
+                to.rng = from.rng;
+        }
+
         /* A pending inelastic DEL, src/pumas.c:5339-5386. */
         PG_FN void walker_del(Walker & w) const
         {
@@ -2136,14 +2194,16 @@ struct EngineT {
                 /* Pre and post DEL points when recording, src/pumas.c:
                  * 5343-5387: the pre point is the state after the DEL with
                  * its energy and direction before it. */
-                const int rec_del = w.record && (rec.period > 0);
+                const int rec_del = !LEAN && w.record && (rec.period > 0);
                 const double ki = t.energy;
                 const double ui[3] = { t.dir[0], t.dir[1], t.dir[2] };
                 {
-                        Track tmp = t;
-                        const EngineT cold = *this;
-                        cold.transport_do_del(tmp, w.material);
-                        t = tmp;
+                        /* The members that the DEL reads or changes. */
+                        Track tmp;
+                        del_members(tmp, t);
+                        const EngineT engine = *this;
+                        engine.transport_do_del(tmp, w.material);
+                        del_members(t, tmp);
                 }
                 if (rec_del) {
                         Walker pre = w;

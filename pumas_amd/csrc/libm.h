@@ -513,14 +513,9 @@ LM_FN double cos(double x)
  * different ranges evaluate the two series together instead of once per
  * range; each lane's operations are those of its range.
  */
-LM_FN void sincos(double x, double * sx, double * cx)
+LM_FN void sincos_near(double x, double * sx, double * cx)
 {
         const uint32_t k = (uint32_t)(asu64(x) >> 32) & 0x7fffffff;
-        if (k >= 0x419921FB) {
-                *sx = sin_far(x);
-                *cx = cos_far(x);
-                return;
-        }
         if (k < 0x3e400000) {
                 *sx = x;
                 *cx = 1.0;
@@ -551,6 +546,18 @@ LM_FN void sincos(double x, double * sx, double * cx)
                 *sx = (n & 2) ? -rs : rs;
                 *cx = ((n + 1) & 2) ? -rc : rc;
         }
+}
+
+/* Any argument (sincos_near: |x| < 105414350, the reductions above). */
+LM_FN void sincos(double x, double * sx, double * cx)
+{
+        const uint32_t k = (uint32_t)(asu64(x) >> 32) & 0x7fffffff;
+        if (k >= 0x419921FB) {
+                *sx = sin_far(x);
+                *cx = cos_far(x);
+                return;
+        }
+        sincos_near(x, sx, cx);
 }
 
 /* ------------------------------------------------------------------------

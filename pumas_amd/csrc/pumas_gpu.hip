@@ -778,10 +778,10 @@ struct KernelArgs {
         int32_t * rc;
         int max_steps;
         int ehs_batch;
-        uint32_t tail_del_lanes; /* resident lanes of the stepping launch */
+        uint32_t resident_lanes; /* of the stepping launch */
         int lanes_per_wave;      /* lanes of a wavefront taking histories */
         int lanes_auto;          /* fewer in the rounds that fit (k_step) */
-        int tail_adaptive;       /* in-wavefront DELs chosen per round */
+        int tail_del;            /* as pumas_gpu_options.tail_del */
         Recorder rec;
         unsigned long long * counters;
         Walker * records;     /* [n] histories in flight */
@@ -827,12 +827,14 @@ __device__ __forceinline__ void walker_load(const KernelArgs & a, uint64_t i,
         t.max_steps = a.max_steps;
 }
 
-/* Store the end state of history i at `s` and its outputs. */
+/* Store the end state of history i at `s` and its outputs. `cold` holds the
+ * members that a lean engine leaves in the record (`w` itself otherwise). */
 __device__ __forceinline__ void walker_store(const KernelArgs & a, uint64_t i,
-    const Walker & w, struct pumas_state * s)
+    const Walker & w, const Walker & cold, struct pumas_state * s)
 {
         const Track & t = w.t;
-        s->charge = t.charge;
+        const int rc = cold.rc;
+        s->charge = cold.t.charge;
         s->energy = t.energy;
         s->distance = t.distance;
         s->grammage = t.grammage;
@@ -844,21 +846,65 @@ __device__ __forceinline__ void walker_store(const KernelArgs & a, uint64_t i,
         s->direction[0] = t.dir[0];
         s->direction[1] = t.dir[1];
         s->direction[2] = t.dir[2];
-        s->decayed = t.decayed;
-        if (a.events) a.events[i] = (enum pumas_event)w.event;
+        s->decayed = cold.t.decayed;
+        if (a.events) a.events[i] = (enum pumas_event)cold.event;
         if (a.media) {
-                a.media[2 * i] = w.media0;
-                a.media[2 * i + 1] = w.end_medium;
+                a.media[2 * i] = cold.media0;
+                a.media[2 * i + 1] = cold.end_medium;
         }
         if (a.steps) a.steps[i] = t.steps;
         if (a.draws) a.draws[i] = t.rng.count;
-        if (a.rc) a.rc[i] = w.rc;
-        if (w.rc >= HISTORY_STEP_LIMIT)
-                atomicAdd(a.counters + C_STATUS + (w.rc - HISTORY_STEP_LIMIT),
+        if (a.rc) a.rc[i] = rc;
+        if (rc >= HISTORY_STEP_LIMIT)
+                atomicAdd(a.counters + C_STATUS + (rc - HISTORY_STEP_LIMIT),
                     1ull);
-        else if (w.rc != RETURN_SUCCESS)
-                atomicCAS(a.counters + C_ERROR, 0ull,
-                    (unsigned long long)w.rc);
+        else if (rc != RETURN_SUCCESS)
+                atomicCAS(a.counters + C_ERROR, 0ull, (unsigned long long)rc);
+}
+
+/* Write a history back to its record; of a lean engine, only the members
+ * that it keeps in registers. */
+template <bool F32, bool LEAN>
+__device__ __forceinline__ void walker_save(Walker * r, const Walker & w)
+{
+        if constexpr (!LEAN) {
+                *r = w;
+                return;
+        }
+        r->t.energy = w.t.energy;
+        r->t.distance = w.t.distance;
+        r->t.grammage = w.t.grammage;
+        r->t.time = w.t.time;
+        r->t.weight = w.t.weight;
+        for (int i = 0; i < 3; i++) {
+                r->t.pos[i] = w.t.pos[i];
+                r->t.dir[i] = w.t.dir[i];
+        }
+        r->t.step_first = w.t.step_first;
+        r->t.step_event = w.t.step_event;
+        r->t.step_foreseen = w.t.step_foreseen;
+        r->t.step_invlb1 = w.t.step_invlb1;
+        r->t.randn_done = w.t.randn_done;
+        r->t.randn_next = w.t.randn_next;
+        r->t.ix = w.t.ix;
+        if constexpr (F32) r->t.fx = w.t.fx;
+        r->t.rng.count = w.t.rng.count;
+        r->t.rng.next_lo = w.t.rng.next_lo;
+        r->t.rng.next_hi = w.t.rng.next_hi;
+        r->t.steps = w.t.steps;
+        r->t.max_steps = w.t.max_steps;
+        r->phase = w.phase;
+        r->medium = w.medium;
+        r->material = w.material;
+        r->straight = w.straight;
+        r->step_index = w.step_index;
+        r->step_max_type = w.step_max_type;
+        r->density = w.density;
+        r->step_max_medium = w.step_max_medium;
+        r->step_max_locals = w.step_max_locals;
+        r->ti = w.ti;
+        r->dei = w.dei;
+        r->grammage_max = w.grammage_max;
 }
 
 __device__ __forceinline__ uint64_t lanes_below()
@@ -966,7 +1012,7 @@ __global__ void __launch_bounds__(INIT_BLOCK)
                 walker_load(a, i, w, stage + threadIdx.x);
                 eng.template walker_init<CLOSED>(w);
                 if (w.phase == PHASE_DONE)
-                        walker_store(a, i, w, stage + threadIdx.x);
+                        walker_store(a, i, w, w, stage + threadIdx.x);
                 if (!CLOSED && (w.phase == PHASE_STEP)) a.records[i] = w;
         }
         __syncthreads();
@@ -1008,16 +1054,47 @@ __global__ void k_round(unsigned long long * c, int parity)
         }
 }
 
+/* The kernel arguments at `args` (the kernarg segment), the same for every
+ * lane: in scalar registers, so that their members are scalar loads also in
+ * out-of-line code. */
+__device__ __forceinline__ const KernelArgs & uniform_args(
+    const KernelArgs * args)
+{
+        typedef const __attribute__((address_space(4))) KernelArgs cargs;
+        const uint64_t v = (uint64_t)args;
+        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+        const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+        return *(const KernelArgs *)(cargs *)(((uint64_t)hi << 32) | lo);
+}
+
+/* The pending DELs of a stepping wavefront's histories, on their records.
+ * Out of line: the DEL samplers are the largest code of the path. */
+template <bool F32>
+__device__ __noinline__ void del_wave(
+    const KernelArgs * args, uint32_t slot, bool pending)
+{
+        const KernelArgs & a = uniform_args(args);
+        if (!pending) return;
+        const EngineT<F32> eng = { a.p, a.mv, a.c, a.g, a.ft, a.p, a.rec };
+        Walker w = a.records[slot];
+        eng.walker_del(w);
+        a.records[slot] = w;
+}
+
 /*
- * Stepping: persistent over the step queue of round `parity`. With
- * TAIL_DEL, a wavefront that can no longer refill (the step queue is
- * exhausted) applies the DELs of its histories itself instead of queueing
- * them for the next round: the last histories of a batch then run to their
- * end without a round barrier per DEL, which sets the latency of small
- * batches. The out-of-line DEL call costs registers on every step, so
- * rounds that fill the device use the variant without it.
+ * Stepping: persistent over the step queue of round `parity`. In a round that
+ * fits in the resident lanes (or always, a.tail_del > 0) a wavefront that can
+ * no longer refill applies the DELs of its histories itself instead of
+ * queueing them for the next round: the last histories of a batch, and small
+ * batches, then run to their end without a round barrier per DEL.
+ *
+ * The DELs run outside of the stepping loop, on the records: the wavefront
+ * saves its histories, calls the DEL code and reloads them, so that nothing
+ * of the stepping loop is live in registers across the call. With the call
+ * inside the loop the kernel spilled 200 to 1400 registers on every step
+ * (12 to 18 without it).
  */
-template <bool F32, bool TAIL_DEL, bool LDS>
+template <bool F32, bool LDS, bool LEAN, int SCHEME>
 __global__ void __launch_bounds__(512, 2) k_step(KernelArgs args, int parity)
 {
         KERNEL_ARGS(args);
@@ -1038,19 +1115,12 @@ __global__ void __launch_bounds__(512, 2) k_step(KernelArgs args, int parity)
                 st = &a.stl;
         else
                 st = &a.p;
-        const EngineT<F32, FT, ST> eng = { a.p, a.mv, a.c, a.g, *ft, *st,
-                a.rec };
+        const EngineT<F32, FT, ST, LEAN, SCHEME> eng = { a.p, a.mv, a.c, a.g,
+                *ft, *st, a.rec, a.records };
         const uint64_t below = lanes_below();
         const uint32_t * in = a.q_step[parity];
         const unsigned long long n_in = a.counters[C_STEP_N0 + parity];
         if (n_in == 0) return;
-        /* Adaptive DEL mode: both variants are launched every round and
-         * the one that does not fit the round's queue returns at once. The
-         * in-wavefront DEL call costs registers on every step, so rounds
-         * that fill the resident lanes run without it; the last rounds of
-         * a batch, and small batches, run with it. */
-        if (a.tail_adaptive && (TAIL_DEL != (n_in <= a.tail_del_lanes)))
-                return;
         if constexpr (LDS) {
                 /* The copy (tens of KB to 160 KB, read from L2 by every
                  * block of the launch), in 16 B words. */
@@ -1064,100 +1134,143 @@ __global__ void __launch_bounds__(512, 2) k_step(KernelArgs args, int parity)
                 }
                 __syncthreads();
         }
-        Walker w;
-        w.phase = PHASE_EMPTY;
         uint32_t slot = 0;
         bool exhausted = false;
-        /* Lanes of the wavefront that take histories. */
-        int lanes = a.lanes_per_wave;
-        if (n_in <= a.tail_del_lanes) {
-                /* The round fits in the resident lanes: each wavefront takes
-                 * its share of the queue once, and the queue has nothing
-                 * more for it. (Taken from the shared counter instead, a
-                 * wavefront learns that only when it asks again, with a
-                 * lane freed by its first DEL: with one history per
-                 * wavefront every DEL cost a round.) The shares are spread
-                 * over all wavefronts, first over the blocks, then over the
-                 * wavefronts of a block, unless the caller asked for a
-                 * number of lanes. */
-                const uint32_t waves =
-                    gridDim.x * (blockDim.x >> 6);
-                if (a.lanes_auto)
-                        lanes = (int)((n_in + waves - 1) / waves);
-                const uint32_t wave =
-                    (threadIdx.x >> 6) * gridDim.x + blockIdx.x;
-                const unsigned long long k =
-                    (unsigned long long)wave * lanes + (threadIdx.x & 63);
-                if (((int)(threadIdx.x & 63) < lanes) && (k < n_in)) {
-                        slot = in[k];
-                        w = a.records[slot];
-                }
-                exhausted = true;
-        }
+        /* A round that fits in the resident lanes: each wavefront takes its
+         * share of the queue once, and the queue has nothing more for it.
+         * (Taken from the shared counter instead, a wavefront learns that
+         * only when it asks again, with a lane freed by its first DEL: with
+         * one history per wavefront every DEL cost a round.) The shares are
+         * spread over all wavefronts, first over the blocks, then over the
+         * wavefronts of a block, unless the caller asked for a number of
+         * lanes. */
+        const bool fits = n_in <= a.resident_lanes;
+        const uint32_t waves = gridDim.x * (blockDim.x >> 6);
+        const int lanes = (fits && a.lanes_auto) ?
+            (int)((n_in + waves - 1) / waves) :
+            a.lanes_per_wave;
         const bool lane_on = (int)(threadIdx.x & 63) < lanes;
+        const bool tail_del = (a.tail_del > 0) || ((a.tail_del == 0) && fits);
         unsigned long long steps_acc = 0;
-        for (;;) {
-                /* Hand over the histories that left the stepping phase. */
-                const bool done = w.phase == PHASE_DONE;
-                const bool to_del =
-                    (w.phase == PHASE_DEL) && !(TAIL_DEL && exhausted);
-                if (done) {
-                        walker_store(a, slot, w, a.states + slot);
-                        steps_acc += w.t.steps;
-                }
-                if (to_del) a.records[slot] = w;
-                queue_append(a.counters + C_DEL_N, a.q_del, to_del, slot);
-                if (done || to_del) w.phase = PHASE_EMPTY;
+        bool held = false; /* the lane has a history, saved in its record */
+        uint64_t del_mask = 0; /* lanes with a DEL to apply here */
+        bool finished = false;
+        do {
+                Walker w;
+                w.phase = PHASE_EMPTY;
+                if (held) w = a.records[slot];
+                for (;;) {
+                        /* Hand over the histories that left the stepping
+                         * phase. */
+                        const bool done = w.phase == PHASE_DONE;
+                        const bool del = w.phase == PHASE_DEL;
+                        if (done) {
+                                if constexpr (LEAN)
+                                        walker_store(a, slot, w,
+                                            a.records[slot], a.states + slot);
+                                else
+                                        walker_store(a, slot, w, w,
+                                            a.states + slot);
+                                steps_acc += w.t.steps;
+                        }
+                        const bool to_del = del && !(tail_del && exhausted);
+                        const uint64_t dels = __ballot(del && !to_del);
+                        const bool save = to_del ||
+                            (dels && (w.phase != PHASE_EMPTY) && !done);
+                        if (save)
+                                walker_save<F32, LEAN>(a.records + slot, w);
+                        queue_append(
+                            a.counters + C_DEL_N, a.q_del, to_del, slot);
+                        if (dels) {
+                                /* DELs in the wavefront, below. */
+                                held = save && !to_del;
+                                del_mask = dels;
+                                break;
+                        }
+                        if (done || to_del) w.phase = PHASE_EMPTY;
 
-                /* Refill the free lanes from the step queue. */
-                if (!exhausted) {
-                        const uint64_t free_lanes =
-                            __ballot((w.phase == PHASE_EMPTY) && lane_on);
-                        if (free_lanes) {
-                                const int count = __popcll(free_lanes);
-                                const int leader = __ffsll(
-                                    (unsigned long long)free_lanes) - 1;
-                                unsigned long long base = 0;
-                                if ((int)(threadIdx.x & 63) == leader)
-                                        base = atomicAdd(
-                                            a.counters + C_TAKEN, count);
-                                base = __shfl(base, leader, 64);
-                                if (base + count >= n_in) exhausted = true;
-                                if ((w.phase == PHASE_EMPTY) && lane_on) {
-                                        const unsigned long long k = base +
-                                            __popcll(free_lanes & below);
-                                        if (k < n_in) {
-                                                slot = in[k];
-                                                w = a.records[slot];
+                        /* Refill the free lanes from the step queue. */
+                        if (!exhausted) {
+                                const uint64_t free_lanes = __ballot(
+                                    (w.phase == PHASE_EMPTY) && lane_on);
+                                if (free_lanes) {
+                                        const int count = __popcll(free_lanes);
+                                        unsigned long long base = 0;
+                                        if (fits) {
+                                                base = (unsigned long long)
+                                                    lanes *
+                                                    ((threadIdx.x >> 6) *
+                                                            gridDim.x +
+                                                        blockIdx.x);
+                                                exhausted = true;
+                                        } else {
+                                                const int leader =
+                                                    __ffsll((unsigned long
+                                                        long)free_lanes) - 1;
+                                                if ((int)(threadIdx.x & 63) ==
+                                                    leader)
+                                                        base = atomicAdd(
+                                                            a.counters +
+                                                                C_TAKEN,
+                                                            count);
+                                                base = __shfl(
+                                                    base, leader, 64);
+                                                if (base + count >= n_in)
+                                                        exhausted = true;
+                                        }
+                                        if ((w.phase == PHASE_EMPTY) &&
+                                            lane_on) {
+                                                const unsigned long long k =
+                                                    base +
+                                                    __popcll(
+                                                        free_lanes & below);
+                                                if (k < n_in) {
+                                                        slot = in[k];
+                                                        w = a.records[slot];
+                                                }
                                         }
                                 }
                         }
-                }
-                if (!__ballot((w.phase == PHASE_STEP) ||
-                        (w.phase == PHASE_EHS) ||
-                        (TAIL_DEL && (w.phase == PHASE_DEL)))) {
-                        if (exhausted) break;
-                        continue;
-                }
-                if (w.phase == PHASE_STEP) eng.walker_step(w);
+                        if (!__ballot((w.phase == PHASE_STEP) ||
+                                (w.phase == PHASE_EHS))) {
+                                if (exhausted) {
+                                        finished = true;
+                                        break;
+                                }
+                                continue;
+                        }
+                        if constexpr (LEAN) {
+                                /* In scalar registers: the same for every
+                                 * history. */
+                                w.t.rng.k0 = (uint32_t)a.seed;
+                                w.t.rng.k1 = (uint32_t)(a.seed >> 32);
+                                w.t.rng.stream = STREAM_TRANSPORT;
+                                w.slot = slot;
+                        }
+                        if (w.phase == PHASE_STEP) eng.walker_step(w);
 
-                /* Elastic hard scatterings, on ~16% of the steps of a muon
-                 * in rock, run once enough lanes wait for one (half of the
-                 * lanes in flight, at most a.ehs_batch) or none can step, so
-                 * that the wavefront runs that code with most lanes busy. */
-                const uint64_t ehs = __ballot(w.phase == PHASE_EHS);
-                const uint64_t stepping = __ballot(w.phase == PHASE_STEP);
-                const int waiting = __popcll(ehs);
-                const int in_flight = waiting + __popcll(stepping);
-                const int batch = (in_flight + 1) / 2 < a.ehs_batch ?
-                    (in_flight + 1) / 2 :
-                    a.ehs_batch;
-                if (ehs && ((waiting >= batch) || !stepping)) {
-                        if (w.phase == PHASE_EHS) eng.walker_ehs(w);
+                        /* Elastic hard scatterings, on ~16% of the steps of
+                         * a muon in rock, run once enough lanes wait for one
+                         * (half of the lanes in flight, at most a.ehs_batch)
+                         * or none can step, so that the wavefront runs that
+                         * code with most lanes busy. */
+                        const uint64_t ehs = __ballot(w.phase == PHASE_EHS);
+                        const uint64_t stepping =
+                            __ballot(w.phase == PHASE_STEP);
+                        const int waiting = __popcll(ehs);
+                        const int in_flight = waiting + __popcll(stepping);
+                        const int batch =
+                            (in_flight + 1) / 2 < a.ehs_batch ?
+                            (in_flight + 1) / 2 :
+                            a.ehs_batch;
+                        if (ehs && ((waiting >= batch) || !stepping)) {
+                                if (w.phase == PHASE_EHS) eng.walker_ehs(w);
+                        }
                 }
-                if (TAIL_DEL && exhausted && (w.phase == PHASE_DEL))
-                        eng.walker_del(w);
-        }
+                if (!finished)
+                        del_wave<F32>(
+                            &a, slot, (del_mask >> (threadIdx.x & 63)) & 1);
+        } while (!finished);
         steps_flush(a, steps_acc);
 }
 
@@ -1187,7 +1300,7 @@ __global__ void __launch_bounds__(256, 2) k_del(KernelArgs args, int parity)
                         w = a.records[slot];
                         eng.walker_del(w);
                         if (w.phase == PHASE_DONE) {
-                                walker_store(a, slot, w, a.states + slot);
+                                walker_store(a, slot, w, w, a.states + slot);
                                 steps_acc += w.t.steps;
                         } else {
                                 a.records[slot] = w;
@@ -1232,7 +1345,7 @@ constexpr int MAX_ROUNDS_PER_CHECK = 256;
 struct Launch {
         int n_cu, block, per_cu, rounds_per_check;
         bool graph;
-        int tail_del; /* <0 never, >0 always, 0: rounds below the lanes */
+        int tail_del; /* <0 never, >0 always, 0: rounds that fit */
         int lanes_per_wave; /* 1..64, or 0: spread small batches */
         unsigned lds_bytes; /* LDS copy of the step tables, or 0 */
         unsigned step_grid, del_grid;
@@ -1242,16 +1355,36 @@ struct Launch {
         bool closed; /* every history takes the closed form CSDA */
 };
 
-template <bool F32, bool TAIL_DEL>
+/* The stepping kernel of a launch. The lean kernels, compiled for one energy
+ * loss mode, serve the launches without a frame recorder whose step tables
+ * fit in LDS; the general one the others (recorders, launch shapes with
+ * several LDS copies per CU, transport without energy loss). Compiled for any
+ * mode, the lean FP64 kernel with in-wavefront DELs spilled 1014 registers
+ * instead of 200. */
+using StepKernel = void (*)(KernelArgs, int);
+
+template <bool F32>
+StepKernel step_kernel(const KernelArgs & a, bool lds)
+{
+        if (!lds) return k_step<F32, false, false, SCHEME_ANY>;
+        if (a.rec.frames) return k_step<F32, true, false, SCHEME_ANY>;
+        switch (a.c.energy_loss) {
+        case MODE_STRAGGLED:
+                return k_step<F32, true, true, MODE_STRAGGLED>;
+        case MODE_MIXED:
+                return k_step<F32, true, true, MODE_MIXED>;
+        case MODE_CSDA:
+                return k_step<F32, true, true, MODE_CSDA>;
+        default:
+                return k_step<F32, true, false, SCHEME_ANY>;
+        }
+}
+
+template <bool F32>
 void launch_step(const KernelArgs & a, int parity, const Launch & L)
 {
-        if (L.lds_bytes)
-                hipLaunchKernelGGL((k_step<F32, TAIL_DEL, true>),
-                    dim3(L.step_grid), dim3(L.block), L.lds_bytes, L.stream,
-                    a, parity);
-        else
-                hipLaunchKernelGGL((k_step<F32, TAIL_DEL, false>),
-                    dim3(L.step_grid), dim3(L.block), 0, L.stream, a, parity);
+        hipLaunchKernelGGL(step_kernel<F32>(a, L.lds_bytes > 0),
+            dim3(L.step_grid), dim3(L.block), L.lds_bytes, L.stream, a, parity);
 }
 
 template <bool F32>
@@ -1262,8 +1395,7 @@ enum pumas_return launch_round(
         hipLaunchKernelGGL(k_round, dim3(1), dim3(64), 0, stream, a.counters,
             parity);
         if (L.marks) HIP_TRY(hipEventRecord(L.marks[2 * r], stream));
-        if (L.tail_del <= 0) launch_step<F32, false>(a, parity, L);
-        if (L.tail_del >= 0) launch_step<F32, true>(a, parity, L);
+        launch_step<F32>(a, parity, L);
         if (L.marks) HIP_TRY(hipEventRecord(L.marks[2 * r + 1], stream));
         hipLaunchKernelGGL(k_del<F32>, dim3(L.del_grid), dim3(256), 0,
             stream, a, parity);
@@ -1271,12 +1403,9 @@ enum pumas_return launch_round(
         return PUMAS_RETURN_SUCCESS;
 }
 
-template <bool F32>
-enum pumas_return allow_lds(int bytes)
+enum pumas_return allow_lds(StepKernel kernel, int bytes)
 {
-        HIP_TRY(hipFuncSetAttribute((const void *)k_step<F32, true, true>,
-            hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
-        HIP_TRY(hipFuncSetAttribute((const void *)k_step<F32, false, true>,
+        HIP_TRY(hipFuncSetAttribute((const void *)kernel,
             hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
         return PUMAS_RETURN_SUCCESS;
 }
@@ -1284,7 +1413,7 @@ enum pumas_return allow_lds(int bytes)
 /* Bytes of the LDS copy of the step tables in the stepping kernel, or 0
  * when `per_cu` copies do not fit in the LDS of a CU. */
 enum pumas_return lds_tables_size(const pumas_gpu_physics * physics,
-    int device, int per_cu, bool f32, unsigned * bytes)
+    const KernelArgs & a, int device, int per_cu, bool f32, unsigned * bytes)
 {
         *bytes = 0;
         const size_t need = f32 ?
@@ -1300,9 +1429,10 @@ enum pumas_return lds_tables_size(const pumas_gpu_physics * physics,
         if ((need > (size_t)per_block) || (need * per_cu > (size_t)per_sm))
                 return PUMAS_RETURN_SUCCESS;
         if (need > 65536) {
-                const enum pumas_return rc = f32 ?
-                    allow_lds<true>((int)need) :
-                    allow_lds<false>((int)need);
+                const enum pumas_return rc = allow_lds(f32 ?
+                        step_kernel<true>(a, true) :
+                        step_kernel<false>(a, true),
+                    (int)need);
                 if (rc != PUMAS_RETURN_SUCCESS) return rc;
         }
         *bytes = (unsigned)need;
@@ -1361,8 +1491,8 @@ enum pumas_return transport_chunk(const KernelArgs & a0, size_t base,
         KernelArgs a = a0;
         a.lanes_per_wave = lanes;
         a.lanes_auto = lanes_auto;
-        a.tail_del_lanes = L.step_grid * (uint32_t)(waves * lanes);
-        a.tail_adaptive = (L.tail_del == 0);
+        a.resident_lanes = L.step_grid * (uint32_t)(waves * lanes);
+        a.tail_del = L.tail_del;
         a.states = a0.states + base;
         a.n = m;
         a.first = a0.first + base;
@@ -1663,7 +1793,8 @@ static enum pumas_return transport_impl(const pumas_gpu_physics * physics,
         const bool f32 = (precision == PUMAS_GPU_PRECISION_FP32_BULK);
         unsigned lds_bytes = 0;
         if (!(options && options->lds_tables < 0)) {
-                rc = lds_tables_size(physics, device, per_cu, f32, &lds_bytes);
+                rc = lds_tables_size(
+                    physics, a, device, per_cu, f32, &lds_bytes);
                 if (rc != PUMAS_RETURN_SUCCESS) return rc;
         }
         unsigned long long total_steps = 0, error = 0;
