@@ -302,10 +302,10 @@ struct pumas_gpu_options {
         int ehs_batch;
         /* Frame recorder, or NULL (see below). */
         const struct pumas_gpu_recorder * recorder;
-        /* DELs of the last histories of a batch applied inside the
-         * stepping wavefronts instead of in queued rounds: > 0 always,
-         * < 0 never, 0 in the rounds whose histories fit in the resident
-         * lanes at once (small requests, and the end of large batches). */
+        /* DELs applied inside the stepping wavefronts instead of in queued
+         * rounds: > 0 always, < 0 never, 0 in the rounds of at most four
+         * times as many histories as resident lanes (small requests, and
+         * the end of large batches). */
         int tail_del;
         /* Tables of the per-step lookups (the FP32 mirrors in FP32-bulk,
          * the FP64 step tables otherwise) read by the stepping kernel from

@@ -731,8 +731,9 @@ extern "C" enum pumas_return pumas_gpu_geometry_create(
  *           the histories go back to the next round's step queue.
  * EHS vertices (~16% of the steps of a muon in rock) are batched inside the
  * stepping wavefront: lanes that reach one wait until enough others do.
- * DEL vertices (~0.2% of the steps at a 5% cutoff) leave the wavefront: the
- * DEL samplers are the largest code of the path (exact DCS models, polar
+ * DEL vertices (~0.2% of the steps at a 5% cutoff) leave the wavefront in the
+ * rounds of large batches, and leave the stepping loop in the other rounds:
+ * the DEL samplers are the largest code of the path (exact DCS models, polar
  * angles, rejection loops) and would hold the stepping kernel's registers
  * for every step. A history's operations are the reference's, in its
  * order; only the interleaving across histories differs, and the random
@@ -779,6 +780,8 @@ struct KernelArgs {
         int max_steps;
         int ehs_batch;
         uint32_t resident_lanes; /* of the stepping launch */
+        uint64_t wave_del_max;   /* histories of a round up to which DELs are
+                                    applied in the wavefronts */
         int lanes_per_wave;      /* lanes of a wavefront taking histories */
         int lanes_auto;          /* fewer in the rounds that fit (k_step) */
         int tail_del;            /* as pumas_gpu_options.tail_del */
@@ -1054,6 +1057,37 @@ __global__ void k_round(unsigned long long * c, int parity)
         }
 }
 
+/*
+ * Schedule of the stepping rounds. Slabs forward FP64, and the same with
+ * backward voxels (1 % cutoff, a DEL every 20 steps), 256 CUs x 512 lanes.
+ *
+ * WAVE_DEL_ROUNDS: a round of at most so many times the resident lanes has its
+ * DELs in the wavefronts, so that it ends the batch; a larger one queues them
+ * for a kernel that runs 64 of them per wavefront. 1 (and queued until the
+ * step queue is exhausted): 2x10^5 muons 147 ms, 10^6 354, 3x10^6 809, voxels
+ * 10^6 121; 2: 74, 324, 782, 119; 4: 77, 306, 775, 121; 8: 77, 292, 771, 139.
+ * DEL_BATCH, DEL_WAIT: such DELs run when so many lanes, or as many as the
+ * others in flight, wait for one, or after so many steps of the others, as
+ * one lane's DEL costs the wavefront as much as many lanes'. At once: voxels
+ * 5x10^4 35.9 ms, terrain 10^5 62.1; 8, 32: 27.6, 55.7; 24, 48: 26.6, 55.9.
+ * HAND_OVER: in a larger round, a wavefront with fewer than so many of 64
+ * lanes left, once the step queue is exhausted, puts its histories in the next
+ * round's queue, instead of stepping them until the last one ends: 0: 10^6
+ * muons 379 ms, voxels 10^6 179, terrain 6x10^5 200; 32: 354, 128, 137; 48:
+ * 377, 126, 131. Not before HAND_OVER_AFTER steps, so that every round makes
+ * progress.
+ * PACK_LANES: a round that fits with more than so many lanes per wavefront, and
+ * in half of the wavefronts of each 512 lane block, is put in that half: one
+ * wavefront per SIMD with twice the lanes. 30011 muons 48.2 -> 45.2 ms, 60000
+ * 53.4 -> 48.6; below it loses: 3000 29.8 -> 32.7, 10000 38.6 -> 40.6.
+ */
+constexpr uint64_t WAVE_DEL_ROUNDS = 4;
+constexpr int DEL_BATCH = 24;
+constexpr int DEL_WAIT = 48;
+constexpr int HAND_OVER = 40;
+constexpr int HAND_OVER_AFTER = 32;
+constexpr uint32_t PACK_LANES = 8;
+
 /* The kernel arguments at `args` (the kernarg segment), the same for every
  * lane: in scalar registers, so that their members are scalar loads also in
  * out-of-line code. */
@@ -1082,11 +1116,11 @@ __device__ __noinline__ void del_wave(
 }
 
 /*
- * Stepping: persistent over the step queue of round `parity`. In a round that
- * fits in the resident lanes (or always, a.tail_del > 0) a wavefront that can
- * no longer refill applies the DELs of its histories itself instead of
- * queueing them for the next round: the last histories of a batch, and small
- * batches, then run to their end without a round barrier per DEL.
+ * Stepping: persistent over the step queue of round `parity`. In a round of at
+ * most a.wave_del_max histories (or always, a.tail_del > 0) a wavefront
+ * applies the DELs of its histories itself instead of queueing them for the
+ * next round: the last histories of a batch, and small batches, then run to
+ * their end without a round barrier per DEL.
  *
  * The DELs run outside of the stepping loop, on the records: the wavefront
  * saves its histories, calls the DEL code and reloads them, so that nothing
@@ -1145,21 +1179,28 @@ __global__ void __launch_bounds__(512, 2) k_step(KernelArgs args, int parity)
          * wavefronts of a block, unless the caller asked for a number of
          * lanes. */
         const bool fits = n_in <= a.resident_lanes;
-        const uint32_t waves = gridDim.x * (blockDim.x >> 6);
+        uint32_t waves = gridDim.x * (blockDim.x >> 6);
+        if ((blockDim.x == 512) && (n_in > waves * PACK_LANES) &&
+            (n_in <= waves * 32))
+                waves /= 2;
         const int lanes = (fits && a.lanes_auto) ?
             (int)((n_in + waves - 1) / waves) :
             a.lanes_per_wave;
         const bool lane_on = (int)(threadIdx.x & 63) < lanes;
-        const bool tail_del = (a.tail_del > 0) || ((a.tail_del == 0) && fits);
+        const bool wave_del = (a.tail_del > 0) ||
+            ((a.tail_del == 0) && (n_in <= a.wave_del_max));
+        /* Lanes below which the histories left are handed over. */
+        const int keep = (wave_del || fits) ? 0 : (lanes * HAND_OVER) / 64;
         unsigned long long steps_acc = 0;
         bool held = false; /* the lane has a history, saved in its record */
         uint64_t del_mask = 0; /* lanes with a DEL to apply here */
+        int del_wait = 0;
         bool finished = false;
         do {
                 Walker w;
                 w.phase = PHASE_EMPTY;
                 if (held) w = a.records[slot];
-                for (;;) {
+                for (int it = 0;; it++) {
                         /* Hand over the histories that left the stepping
                          * phase. */
                         const bool done = w.phase == PHASE_DONE;
@@ -1173,21 +1214,43 @@ __global__ void __launch_bounds__(512, 2) k_step(KernelArgs args, int parity)
                                             a.states + slot);
                                 steps_acc += w.t.steps;
                         }
-                        const bool to_del = del && !(tail_del && exhausted);
-                        const uint64_t dels = __ballot(del && !to_del);
-                        const bool save = to_del ||
+                        const bool to_del = del && !wave_del;
+                        uint64_t dels = __ballot(del && wave_del);
+                        if (dels) {
+                                const int others = __popcll(
+                                    __ballot((w.phase == PHASE_STEP) ||
+                                        (w.phase == PHASE_EHS)));
+                                const int waiting = __popcll(dels);
+                                if ((waiting < others) &&
+                                    (waiting < DEL_BATCH) &&
+                                    (++del_wait <= DEL_WAIT))
+                                        dels = 0; /* not yet */
+                                else
+                                        del_wait = 0;
+                        }
+                        bool to_step = false;
+                        if (keep && exhausted && (it > HAND_OVER_AFTER)) {
+                                const bool left = (w.phase == PHASE_STEP) ||
+                                    (w.phase == PHASE_EHS);
+                                to_step = left &&
+                                    (__popcll(__ballot(left)) < keep);
+                        }
+                        const bool save = to_del || to_step ||
                             (dels && (w.phase != PHASE_EMPTY) && !done);
                         if (save)
                                 walker_save<F32, LEAN>(a.records + slot, w);
                         queue_append(
                             a.counters + C_DEL_N, a.q_del, to_del, slot);
+                        queue_append(a.counters + C_STEP_N0 + (parity ^ 1),
+                            a.q_step[parity ^ 1], to_step, slot);
                         if (dels) {
                                 /* DELs in the wavefront, below. */
-                                held = save && !to_del;
+                                held = save;
                                 del_mask = dels;
                                 break;
                         }
-                        if (done || to_del) w.phase = PHASE_EMPTY;
+                        if (done || to_del || to_step)
+                                w.phase = PHASE_EMPTY;
 
                         /* Refill the free lanes from the step queue. */
                         if (!exhausted) {
@@ -1345,7 +1408,7 @@ constexpr int MAX_ROUNDS_PER_CHECK = 256;
 struct Launch {
         int n_cu, block, per_cu, rounds_per_check;
         bool graph;
-        int tail_del; /* <0 never, >0 always, 0: rounds that fit */
+        int tail_del; /* <0 never, >0 always, 0: rounds of few histories */
         int lanes_per_wave; /* 1..64, or 0: spread small batches */
         unsigned lds_bytes; /* LDS copy of the step tables, or 0 */
         unsigned step_grid, del_grid;
@@ -1492,6 +1555,7 @@ enum pumas_return transport_chunk(const KernelArgs & a0, size_t base,
         a.lanes_per_wave = lanes;
         a.lanes_auto = lanes_auto;
         a.resident_lanes = L.step_grid * (uint32_t)(waves * lanes);
+        a.wave_del_max = WAVE_DEL_ROUNDS * a.resident_lanes;
         a.tail_del = L.tail_del;
         a.states = a0.states + base;
         a.n = m;

@@ -278,12 +278,15 @@ def test_lanes_per_wave_invariance(gpu_standard, lanes):
         np.testing.assert_array_equal(getattr(alt, k), getattr(ref, k))
 
 
-@pytest.mark.parametrize("n", [1, 255, 257, 16383, 16384, 16385, 33001])
+@pytest.mark.parametrize("n", [1, 255, 257, 16383, 16384, 16385, 33001, 65536,
+                               65537, 140003])
 def test_round_sizes_invariance(gpu_standard, n):
     """A round that fits in the resident lanes (here 256 CUs x one wavefront
     = 16384) shares its histories out over the wavefronts; a larger one
-    hands them out from a counter. Both, and the rounds without discrete
-    losses in the wavefronts, give the same results."""
+    hands them out from a counter, and one of more than four times the lanes
+    queues its discrete losses and hands histories over to the next round.
+    All, and the rounds without discrete losses in the wavefronts, give the
+    same results."""
     s = W.slabs_forward_states(n, seed=18)
     geom = pa.Geometry(gpu_standard, W.slabs_geometry())
     ctx = W.slabs_forward_context()
@@ -294,3 +297,66 @@ def test_round_sizes_invariance(gpu_standard, n):
     assert (alt.states == ref.states).all()
     for k in ("events", "media", "steps", "draws", "rc"):
         np.testing.assert_array_equal(getattr(alt, k), getattr(ref, k))
+
+
+@pytest.mark.parametrize("n", [8 * 2048, 8 * 2048 + 1, 32 * 2048 + 1])
+def test_packed_round_invariance(gpu_standard, n):
+    """A round of more than 8 and at most 32 histories per wavefront takes
+    half of the wavefronts (256 CUs x 8)."""
+    s = W.slabs_forward_states(n, seed=19)
+    geom = pa.Geometry(gpu_standard, W.slabs_geometry())
+    ctx = W.slabs_forward_context()
+    ref = pa.transport(gpu_standard, ctx, geom, s.copy(), seed=19,
+                       lanes_per_wave=64)
+    alt = pa.transport(gpu_standard, ctx, geom, s.copy(), seed=19)
+    assert (alt.states == ref.states).all()
+    for k in ("events", "media", "steps", "draws", "rc"):
+        np.testing.assert_array_equal(getattr(alt, k), getattr(ref, k))
+
+
+@pytest.mark.parametrize("precision", [pa.Precision.FP64,
+                                       pa.Precision.FP32_BULK])
+@pytest.mark.parametrize("forward", [True, False])
+@pytest.mark.parametrize("loss", [pa.Mode.DISABLED, pa.Mode.CSDA,
+                                  pa.Mode.MIXED, pa.Mode.STRAGGLED])
+def test_stepping_kernels_equal_general(gpu_standard, loss, forward,
+                                        precision):
+    """The stepping kernels compiled for one energy loss mode equal the
+    general one (taken with lds_tables < 0, and with a frame recorder), over
+    the decay modes, the limits and events that end a history, scattering,
+    and uniform and exponential media."""
+    E = pa.Event
+    limits = dict(limit_distance=900.0, limit_grammage=8e5, limit_time=1e3,
+                  limit_energy=20.0 if forward else 500.0)
+    every = E.LIMIT_DISTANCE | E.LIMIT_GRAMMAGE | E.LIMIT_TIME
+    forms = [dict(), dict(decay=pa.Mode.RANDOMISED),
+             dict(event=E.LIMIT_ENERGY), dict(event=every),
+             dict(event=every, decay=pa.Mode.RANDOMISED),
+             dict(event=E.MEDIUM), dict(event=E.VERTEX_COULOMB),
+             dict(event=E.VERTEX_DEL | E.LIMIT_DISTANCE),
+             dict(scattering=pa.Mode.DISABLED, event=E.LIMIT_DISTANCE)]
+    if loss == pa.Mode.DISABLED:
+        forms = [f for f in forms if int(f.get("event", 0)) & int(every)]
+    make = W.slabs_forward_states if forward else W.slabs_backward_states
+    base = (W.slabs_forward_context if forward else
+            W.slabs_backward_context)(energy_loss=loss)
+    for k, desc in enumerate((W.slabs_geometry(), W.atmosphere_geometry())):
+        geom = pa.Geometry(gpu_standard, desc)
+        s = make(501, seed=20 + k, **({} if forward else dict(kmax=50.0)))
+        if k and forward:
+            s["position"][:, 2] = 1999.0
+        for form in forms:
+            ctx = base.replace(**{**limits, **form})
+            kw = dict(seed=20, precision=precision, raise_errors=False,
+                      max_steps=20000)
+            lean = pa.transport(gpu_standard, ctx, geom, s.copy(), **kw)
+            hbm = pa.transport(gpu_standard, ctx, geom, s.copy(),
+                               lds_tables=-1, **kw)
+            rec = pa.transport(gpu_standard, ctx, geom, s.copy(),
+                               recorder=pa.Recorder(16, period=0), **kw)
+            assert lean.steps.sum() > 0
+            for other in (hbm, rec):
+                assert (lean.states == other.states).all(), form
+                for f in ("events", "media", "steps", "draws", "rc"):
+                    np.testing.assert_array_equal(
+                        getattr(lean, f), getattr(other, f), str(form))
