@@ -129,3 +129,45 @@ def test_bad_specs():
         pa.tally(s, spec=pa.TallySpec(n_energy_bins=4, energy_min=-1.0))
     with pytest.raises(pa.PumasError):
         pa.tally(s, spec=pa.TallySpec(flux=7))
+
+
+@pytest.mark.parametrize("n", [0, 1, 63, 257, 300_001])
+@pytest.mark.parametrize("n_e,n_c", [(1, 256), (256, 1), (80, 36), (0, 7)])
+def test_sums_in_fixed_order(n, n_e, n_c):
+    """The sums of weights, added on the host in the tally's order: 256 states
+    a chunk, chunks to at most 1024 blocks in turn; a block's bins in index
+    order, its total by thread and then by a pairwise tree; blocks in order.
+    Equal bit for bit."""
+    s = random_states(n, 7)
+    bc = np.arange(n) % max(n_c, 1)
+    be = (np.arange(n) * 7) % max(n_e, 1)
+    s["energy"] = 1.0 + 10.0 * (be + 0.5) / max(n_e, 1)
+    s["direction"][:, 2] = -(0.1 + 0.8 * (bc + 0.5) / max(n_c, 1))
+    # Energy bins are logarithmic: bin of the value, away from the edges.
+    be = np.floor(np.log(s["energy"]) / np.log(12.0) * n_e).astype(int)
+    spec = pa.TallySpec(flux=pa.Flux.NONE, n_energy_bins=n_e, energy_min=1.0,
+                        energy_max=12.0, n_cos_bins=n_c, cos_min=0.1,
+                        cos_max=0.9)
+    t = pa.tally(s, spec=spec)
+    assert t.count == n
+    v = s["weight"]
+    chunk = np.arange(n) // 256
+    grid = max(1, min((n + 255) // 256, 1024))
+    block = chunk % grid
+    # Of a block's values, those of one thread are added in chunk order.
+    threads = np.zeros((grid, 256))
+    np.add.at(threads, (block, np.arange(n) % 256), v)
+    while threads.shape[1] > 1:
+        half = threads.shape[1] // 2
+        threads = threads[:, :half] + threads[:, half:]
+    assert t.sum == sum(threads[:, 0].tolist(), 0.0)
+    for got, bins, b in ((t.energy, n_e, be), (t.cos_theta, n_c, bc)):
+        if bins == 0:
+            continue
+        for k, w in enumerate((v, v * v)):
+            part = np.zeros((grid, bins))
+            np.add.at(part, (block, b), w)
+            total = np.zeros(bins)
+            for row in part:
+                total = total + row
+            assert (got[:, k] == total).all()
