@@ -208,71 +208,178 @@ struct EngineT {
                 return (SCHEME == SCHEME_ANY) ? c.energy_loss : SCHEME;
         }
 
-        /* Per-step table lookups, in the bulk precision. */
+        /* Per-step table lookups at a located energy: interpolations of the
+         * row tables in a lean FP64 engine, else the accessors, in the bulk
+         * precision, at its kinetic energy. */
+        static constexpr bool ROWS = LEAN && !F32;
+
+        PG_FN Located locate(Track & t, int material, double kinetic) const
+        {
+                if constexpr (ROWS) {
+                        return st.locate(material, kinetic, t.ix.k);
+                } else {
+                        Located l = {};
+                        l.kinetic = kinetic;
+                        return l;
+                }
+        }
+
+        /* The first positive energy of the grid. */
+        PG_FN double k_first() const
+        {
+                if constexpr (ROWS)
+                        return st.rows[ROW_COLUMNS + ROW_K];
+                else
+                        return p.K[1];
+        }
+
         PG_FN double bulk_grammage(Track & t, int scheme, int material,
-            double kinetic) const
+            const Located & l) const
         {
                 if constexpr (F32)
                         return fcel_grammage(
-                            ft, t.fx, scheme, material, (float)kinetic);
-                else
-                        return cel_grammage(st, t.ix, scheme, material, kinetic);
+                            ft, t.fx, scheme, material, (float)l.kinetic);
+                else if constexpr (ROWS) {
+                        if (l.side == 0) return st.value(l, ROW_X);
+                        if (l.side < 0) return 0.;
+                        const double a = p.a_max[material];
+                        const double b = b_max(p, scheme, material);
+                        const double K0 = st.last(material, ROW_K);
+                        const double K1 = a / b + p.mass;
+                        return st.last(material, ROW_X) +
+                            1. / b * lm::log((l.kinetic + K1) / (K0 + K1));
+                } else
+                        return cel_grammage(
+                            st, t.ix, scheme, material, l.kinetic);
         }
 
         PG_FN double bulk_energy_loss(Track & t, int scheme, int material,
-            double kinetic) const
+            const Located & l) const
         {
                 if constexpr (F32)
                         return fcel_energy_loss(
-                            ft, t.fx, scheme, material, (float)kinetic);
-                else
+                            ft, t.fx, scheme, material, (float)l.kinetic);
+                else if constexpr (ROWS) {
+                        if (l.side == 0) return st.value(l, ROW_DE);
+                        if (l.side < 0) return 0.;
+                        return p.a_max[material] +
+                            b_max(p, scheme, material) * (l.kinetic + p.mass);
+                } else
                         return cel_energy_loss(
-                            st, t.ix, scheme, material, kinetic);
+                            st, t.ix, scheme, material, l.kinetic);
         }
 
         PG_FN double bulk_straggling(Track & t, int material,
-            double kinetic) const
+            const Located & l) const
         {
                 if constexpr (F32)
                         return fcel_straggling(
-                            ft, t.fx, material, (float)kinetic);
-                else
-                        return cel_straggling(st, t.ix, material, kinetic);
+                            ft, t.fx, material, (float)l.kinetic);
+                else if constexpr (ROWS) {
+                        if (l.side == 0) return st.value(l, ROW_OMEGA);
+                        if (l.side < 0) return 0.;
+                        const double r = (l.kinetic + p.mass) /
+                            (st.last(material, ROW_K) + p.mass);
+                        return st.last(material, ROW_OMEGA) * r * r;
+                } else
+                        return cel_straggling(st, t.ix, material, l.kinetic);
         }
 
         PG_FN double bulk_del_cross_section(Track & t, int material,
-            double kinetic) const
+            const Located & l) const
         {
                 if constexpr (F32)
                         return fdel_cross_section(
-                            ft, t.fx, material, (float)kinetic);
-                else
-                        return del_cross_section(st, t.ix, material, kinetic);
+                            ft, t.fx, material, (float)l.kinetic);
+                else if constexpr (ROWS) {
+                        if (l.side == 0) return st.value(l, ROW_CS);
+                        if (l.side < 0) return 0.;
+                        return st.last(material, ROW_CS);
+                } else
+                        return del_cross_section(
+                            st, t.ix, material, l.kinetic);
         }
 
         PG_FN double bulk_ehs_length(Track & t, int material,
-            double kinetic) const
+            const Located & l) const
         {
                 if constexpr (F32)
                         return fcoulomb_ehs_length(
-                            ft, t.fx, material, (float)kinetic);
-                else
-                        return coulomb_ehs_length(st, t.ix, material, kinetic);
+                            ft, t.fx, material, (float)l.kinetic);
+                else if constexpr (ROWS) {
+                        const double p2 =
+                            l.kinetic * (l.kinetic + 2. * p.mass);
+                        const int c = ROW_LB;
+                        if (l.side > 0) return st.last(material, c) / p2;
+                        if ((l.side < 0) || (l.row == 0))
+                                return st.rows[st.record(material, 1) + c] / p2;
+                        const double l0 = st.rows[l.at + c];
+                        const double l1 = st.rows[l.at + ROW_COLUMNS + c];
+                        return (l0 + l.t * (l1 - l0)) / p2;
+                } else
+                        return coulomb_ehs_length(
+                            st, t.ix, material, l.kinetic);
         }
 
         PG_FN void bulk_msc(Track & t, int scheme, int material,
-            double kinetic, double * mu0, double * invlb1) const
+            const Located & l, double * mu0, double * invlb1) const
         {
                 if constexpr (F32) {
-                        float m, l;
+                        float m, b;
                         ftable_get_msc(ft, t.fx, scheme, material,
-                            (float)kinetic, &m, &l);
+                            (float)l.kinetic, &m, &b);
                         *mu0 = m;
-                        *invlb1 = l;
+                        *invlb1 = b;
+                } else if constexpr (ROWS) {
+                        if (l.side > 0) {
+                                *mu0 = st.last(material, ROW_MU0);
+                                *invlb1 = st.last(material, ROW_MS1) *
+                                    st.last(material, ROW_K) / l.kinetic;
+                        } else if ((l.side < 0) || (l.row == 0)) {
+                                const int at = st.record(material, 1);
+                                *mu0 = st.rows[at + ROW_MU0];
+                                *invlb1 = st.rows[at + ROW_MS1] *
+                                    sqrt(st.rows[at + ROW_K] / l.kinetic);
+                        } else {
+                                *mu0 = st.value(l, ROW_MU0);
+                                *invlb1 = st.value(l, ROW_MS1);
+                        }
                 } else {
-                        table_get_msc(
-                            st, t.ix, scheme, material, kinetic, mu0, invlb1);
+                        table_get_msc(st, t.ix, scheme, material, l.kinetic,
+                            mu0, invlb1);
                 }
+        }
+
+        /* cel_kinetic_energy (src/pumas.c:3758-3784) of the step tables. */
+        PG_FN double bulk_kinetic_energy(Track & t, int scheme, int material,
+            double grammage) const
+        {
+                if constexpr (ROWS) {
+                        const int first = st.record(material, 0);
+                        double x0, x1;
+                        const int i = st.find(
+                            first, ROW_X, grammage, t.ix.k[0], x0, x1);
+                        if (i < 0) return 0.;
+                        if (i >= st.n_energies - 1) {
+                                const double a = p.a_max[material];
+                                const double b = b_max(p, scheme, material);
+                                const double K0 = st.last(material, ROW_K);
+                                const double K1 = a / b + p.mass;
+                                return (K0 + K1) * lm::exp(b * (grammage -
+                                           st.last(material, ROW_X))) - K1;
+                        }
+                        const int at = first + i * ROW_COLUMNS;
+                        const int to = at + ROW_COLUMNS;
+                        const double dX = x1 - x0;
+                        const double u = (grammage - x0) / dX;
+                        const double m1 = st.rows[at + ROW_K_DX] * dX;
+                        const double m2 =
+                            (i > 0) ? st.rows[to + ROW_K_DX] * dX : m1;
+                        return pchip(u, st.rows[at + ROW_K],
+                            st.rows[to + ROW_K], m1, m2);
+                } else
+                        return cel_kinetic_energy(
+                            st, t.ix, scheme, material, grammage);
         }
 
         /* -ln(u) for an exponential path length or angle. */
@@ -706,7 +813,7 @@ struct EngineT {
                 if (foreseen == EVENT_NONE) return;
 
                 const double X = Xi +
-                    s * (Xf - cel_grammage(st, t.ix, scheme, material, kinetic_limit));
+                    s * (Xf - cel_grammage(p, t.ix, scheme, material, kinetic_limit));
                 if ((*grammage_max <= 0) || (X < *grammage_max)) {
                         *grammage_max = X;
                         t.step_foreseen = foreseen;
@@ -714,25 +821,25 @@ struct EngineT {
         }
 
         /* step_fluctuate, src/pumas.c:6943-7005. */
-        PG_FN void step_fluctuate(Track & t, int material, double Xtot,
-            double dX, double * kf, double * ratio) const
+        PG_FN void step_fluctuate(Track & t, int material, const Located & l0,
+            double Xtot, double dX, double * kf, double * ratio) const
         {
                 const int scheme = loss();
                 const double s = sgn();
                 double k1, r = 0.;
-                k1 = cel_kinetic_energy(st, t.ix, scheme, material, Xtot - s * dX);
+                k1 = bulk_kinetic_energy(t, scheme, material, Xtot - s * dX);
                 const double dk0 = fabs(t.energy - k1);
                 if ((k1 > 0.) && (dk0 > 0.)) {
-                        const double Omega0 =
-                            bulk_straggling(t, material, t.energy);
-                        const double Omega1 = bulk_straggling(t, material, k1);
+                        const double Omega0 = bulk_straggling(t, material, l0);
+                        const Located l1 = locate(t, material, k1);
+                        const double Omega1 = bulk_straggling(t, material, l1);
                         double dk12 = 0.5 * dX * (Omega0 + Omega1);
                         const double tmp = dX / Xtot;
                         if (tmp > 5E-02) {
                                 const double de1 =
-                                    bulk_energy_loss(t, scheme, material, k1);
-                                const double de0 = bulk_energy_loss(
-                                    t, scheme, material, t.energy);
+                                    bulk_energy_loss(t, scheme, material, l1);
+                                const double de0 =
+                                    bulk_energy_loss(t, scheme, material, l0);
                                 dk12 *= 1. + s * dX / dk0 * (de1 - de0);
                         }
                         const double dk1 = sqrt(dk12);
@@ -793,8 +900,8 @@ struct EngineT {
 
                 const int tmp_scheme =
                     (scheme == MODE_DISABLED) ? MODE_CSDA : scheme;
-                const double Xtot =
-                    bulk_grammage(t, tmp_scheme, material, t.energy);
+                const Located l0 = locate(t, material, t.energy);
+                const double Xtot = bulk_grammage(t, tmp_scheme, material, l0);
 
                 double step_loc;
                 double invlb1 = 0.;
@@ -812,8 +919,8 @@ struct EngineT {
                         if (c.scattering == MODE_MIXED) {
                                 if (t.step_first != 0) {
                                         double mu0;
-                                        bulk_msc(t, scheme, material,
-                                            t.energy, &mu0, &invlb1);
+                                        bulk_msc(t, scheme, material, l0,
+                                            &mu0, &invlb1);
                                         invlb1 *= density;
                                 } else
                                         invlb1 = t.step_invlb1;
@@ -960,7 +1067,7 @@ struct EngineT {
                                 }
                         } else if (dX < EPSILON_X * Xtot) {
                                 k1 -= sg *
-                                    bulk_energy_loss(t, scheme, material, k1) *
+                                    bulk_energy_loss(t, scheme, material, l0) *
                                     dX;
                                 if ((c.event & EVENT_LIMIT_ENERGY) &&
                                     (c.limit_energy > 0.)) {
@@ -975,11 +1082,11 @@ struct EngineT {
                                         k1 = 0.;
                                 }
                         } else {
-                                k1 = cel_kinetic_energy(st, t.ix, scheme, material, X);
+                                k1 = bulk_kinetic_energy(t, scheme, material, X);
                         }
                 } else if (scheme == MODE_STRAGGLED) {
                         double ratio;
-                        step_fluctuate(t, material, Xtot, dX, &k1, &ratio);
+                        step_fluctuate(t, material, l0, Xtot, dX, &k1, &ratio);
                         dk = fabs(t.energy - k1);
 
                         double kinetic_limit = -1.;
@@ -1012,24 +1119,27 @@ struct EngineT {
                                 if (Xmax > dX1) Xmax = dX1;
                         }
                         double k_x = -1.;
+                        const Located l1 = locate(t, material, k1);
 
                         /* In-step inelastic DEL. */
                         do {
                                 double xs_del =
-                                    bulk_del_cross_section(t, material, t.energy);
+                                    bulk_del_cross_section(t, material, l0);
                                 const double tmp_del =
-                                    bulk_del_cross_section(t, material, k1);
+                                    bulk_del_cross_section(t, material, l1);
                                 if (tmp_del > xs_del) xs_del = tmp_del;
                                 if (xs_del <= 0.) break;
                                 const double X_del =
                                     bulk_neglog_uniform(t) / xs_del;
                                 if (X_del >= Xmax) break;
-                                const double k_h = cel_kinetic_energy(st, t.ix, scheme, material, Xtot - sg * X_del);
+                                const double k_h = bulk_kinetic_energy(
+                                    t, scheme, material, Xtot - sg * X_del);
                                 const double k_del = t.energy -
                                     sg * ratio * fabs(t.energy - k_h);
                                 if (k_del <= 0.) break;
                                 const double r =
-                                    bulk_del_cross_section(t, material, k_del) /
+                                    bulk_del_cross_section(t, material,
+                                        locate(t, material, k_del)) /
                                     xs_del;
                                 if (t.rng.uniform() > r) break;
                                 k_x = k_del;
@@ -1039,27 +1149,26 @@ struct EngineT {
 
                         /* In-step elastic hard scattering. */
                         if (c.scattering == MODE_MIXED) do {
-                                double kmin, kmax;
-                                if (k1 <= t.energy)
-                                        kmin = k1, kmax = t.energy;
-                                else
-                                        kmax = k1, kmin = t.energy;
-                                if (kmin < p.K[1]) {
-                                        const double tmp = kmin;
-                                        kmin = kmax, kmax = tmp;
-                                }
-                                const double lb_ehs =
-                                    bulk_ehs_length(t, material, kmin);
+                                /* At the lower energy, but the higher one
+                                 * when that is in the first row. */
+                                const double kmin =
+                                    (k1 <= t.energy) ? k1 : t.energy;
+                                const bool at_k1 =
+                                    (k1 <= t.energy) != (kmin < k_first());
+                                const double lb_ehs = bulk_ehs_length(
+                                    t, material, at_k1 ? l1 : l0);
                                 if (lb_ehs <= 0.) break;
                                 const double X_ehs =
                                     bulk_neglog_uniform(t) * lb_ehs;
                                 if (X_ehs >= Xmax) break;
-                                const double k_h = cel_kinetic_energy(st, t.ix, scheme, material, Xtot - sg * X_ehs);
+                                const double k_h = bulk_kinetic_energy(
+                                    t, scheme, material, Xtot - sg * X_ehs);
                                 const double k_ehs = t.energy -
                                     sg * ratio * fabs(t.energy - k_h);
                                 if (k_ehs <= 0.) break;
                                 const double r =
-                                    bulk_ehs_length(t, material, k_ehs) /
+                                    bulk_ehs_length(t, material,
+                                        locate(t, material, k_ehs)) /
                                     lb_ehs;
                                 if ((r <= 0.) || (t.rng.uniform() > 1. / r))
                                         break;
@@ -1094,7 +1203,7 @@ struct EngineT {
                         if (!(event & EVENT_LIMIT_ENERGY)) {
                                 if (scheme <= MODE_MIXED) {
                                         if (scheme != MODE_DISABLED)
-                                                k1 = cel_kinetic_energy(st, t.ix,
+                                                k1 = bulk_kinetic_energy(t,
                                                     scheme, material,
                                                     Xtot - sg * (t.grammage -
                                                                     Xi));
@@ -1143,7 +1252,7 @@ struct EngineT {
                                                 t.grammage = Xi + dxT;
                                                 const double xf =
                                                     Xtot - sg * dxT;
-                                                k1 = cel_kinetic_energy(st, t.ix, scheme, material, xf);
+                                                k1 = bulk_kinetic_energy(t, scheme, material, xf);
                                         }
                                 }
                         }
@@ -1212,8 +1321,9 @@ struct EngineT {
                         if (t.energy <= 0.) {
                                 t.step_invlb1 = invlb1;
                         } else {
-                                bulk_msc(t, scheme, material, t.energy,
-                                    &mu0, &invlb1_);
+                                bulk_msc(t, scheme, material,
+                                    locate(t, material, t.energy), &mu0,
+                                    &invlb1_);
                                 t.step_invlb1 = locals_density * invlb1_;
                         }
                 }
@@ -1744,17 +1854,8 @@ struct EngineT {
         {
                 const double kinetic = t.energy;
                 double mu0 = 0., invlb1 = 0.;
-                /* The FP64 step tables (st) hold the MSC columns in FP64
-                 * mode; FP32-bulk reads its single precision mirrors. */
-                if constexpr (F32) {
-                        float m, l;
-                        ftable_get_msc(ft, t.fx, loss(), material,
-                            (float)kinetic, &m, &l);
-                        mu0 = m;
-                        invlb1 = l;
-                } else
-                        table_get_msc(st, t.ix, loss(), material,
-                            kinetic, &mu0, &invlb1);
+                bulk_msc(t, loss(), material, locate(t, material, kinetic),
+                    &mu0, &invlb1);
 
                 const int nc = p.elements_in[material];
                 int ihard = nc - 1;

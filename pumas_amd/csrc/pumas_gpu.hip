@@ -72,6 +72,13 @@ struct LdsStepTables {
         static constexpr bool coarse_index = false;
 };
 
+/* The row tables, the whole LDS copy of the lean FP64 kernels. */
+struct LdsRowColumn {
+        PG_FN double operator[](int i) const { return pg_lds_doubles[i]; }
+};
+
+using LdsRowTables = RowTables<LdsRowColumn>;
+
 /* ------------------------------------------------------------------------
  * Error reporting.
  * ------------------------------------------------------------------------ */
@@ -133,6 +140,10 @@ struct pumas_gpu_physics {
         LdsStepTables lds_range;
         uint32_t range_head;    /* doubles of K..K_dX at the head of step */
         uint32_t range_tail_at; /* a_max..b_max: from here to n_step */
+        /* Row tables of the CSDA [0], and of the mixed and straggled [1]
+         * energy losses, for the lean FP64 kernels' LDS copy. */
+        const double * rows[2];
+        uint32_t n_rows;        /* doubles in each (even) */
         int particle;
 };
 
@@ -258,6 +269,52 @@ extern "C" enum pumas_return pumas_gpu_physics_upload_memory(
                 while (step.size() % 8) step.push_back(0.);
         }
 
+        /* Row tables, by energy loss scheme. */
+        const size_t nK = h.imeta[PTAB_N_ENERGIES];
+        const size_t n_rows = (nM * nK * ROW_COLUMNS + 1) / 2 * 2;
+        std::vector<double> rows(2 * n_rows, 0.);
+        {
+                static const struct {
+                        const char * name;
+                        int column;
+                        int schemes; /* 0: none, else its first scheme */
+                } columns[] = { { "X", ROW_X, 1 }, { "X_dK", ROW_X_DK, 1 },
+                        { "K_dX", ROW_K_DX, 1 }, { "dE", ROW_DE, 1 },
+                        { "dE_dK", ROW_DE_DK, 1 }, { "Omega", ROW_OMEGA, 0 },
+                        { "Omega_dK", ROW_OMEGA_DK, 0 }, { "CS", ROW_CS, 0 },
+                        { "CS_dK", ROW_CS_DK, 0 }, { "Mu0", ROW_MU0, 0 },
+                        { "Mu0_dK", ROW_MU0_DK, 0 }, { "Ms1", ROW_MS1, 2 },
+                        { "Ms1_dK", ROW_MS1_DK, 2 }, { "Lb", ROW_LB, 0 },
+                        { "K", ROW_K, -1 } };
+                for (const auto & col : columns) {
+                        const Section * sec = find(sections, col.name);
+                        const size_t tables = (col.schemes < 0) ? 1 :
+                            (size_t)nM * (col.schemes + 1);
+                        if ((sec == nullptr) || (sec->dtype != PTAB_F64) ||
+                            (sec->count < tables * nK))
+                                return pg_fail(PUMAS_RETURN_FORMAT_ERROR,
+                                    "PTAB section `%s' is missing or short",
+                                    col.name);
+                        const double * src = reinterpret_cast<const double *>(
+                            image + sec->offset);
+                        for (int sch = 0; sch < 2; sch++)
+                                for (int m = 0; m < nM; m++) {
+                                        /* Ms1 holds one more scheme first. */
+                                        const size_t table =
+                                            (col.schemes < 0) ? 0 :
+                                            (col.schemes == 0) ? m :
+                                            (size_t)(sch + col.schemes - 1) *
+                                                nM + m;
+                                        for (size_t i = 0; i < nK; i++)
+                                                rows[sch * n_rows +
+                                                    (m * nK + i) *
+                                                        ROW_COLUMNS +
+                                                    col.column] =
+                                                    src[table * nK + i];
+                                }
+                }
+        }
+
         /* Coarse index of the kinetic energy grid (k_index_fast). */
         std::vector<int16_t> coarse(4096);
         int k_bin0 = 0;
@@ -278,7 +335,9 @@ extern "C" enum pumas_return pumas_gpu_physics_upload_memory(
             floats.size() * sizeof(float) + 255) / 256 * 256;
         const size_t coarse_offset = (step_offset +
             step.size() * sizeof(double) + 255) / 256 * 256;
-        const size_t total = coarse_offset + coarse.size() * sizeof(int16_t);
+        const size_t rows_offset = (coarse_offset +
+            coarse.size() * sizeof(int16_t) + 255) / 256 * 256;
+        const size_t total = rows_offset + rows.size() * sizeof(double);
         void * device = nullptr;
         HIP_TRY(hipMalloc(&device, total));
         hipError_t e1 = hipMemcpy(device, image, size, hipMemcpyHostToDevice);
@@ -293,8 +352,10 @@ extern "C" enum pumas_return pumas_gpu_physics_upload_memory(
         hipError_t e5 = coarse.empty() ? hipSuccess :
             hipMemcpy((uint8_t *)device + coarse_offset, coarse.data(),
                 coarse.size() * sizeof(int16_t), hipMemcpyHostToDevice);
+        hipError_t e6 = hipMemcpy((uint8_t *)device + rows_offset, rows.data(),
+            rows.size() * sizeof(double), hipMemcpyHostToDevice);
         if ((e1 != hipSuccess) || (e2 != hipSuccess) || (e3 != hipSuccess) ||
-            (e4 != hipSuccess) || (e5 != hipSuccess)) {
+            (e4 != hipSuccess) || (e5 != hipSuccess) || (e6 != hipSuccess)) {
                 (void)hipFree(device);
                 return pg_fail(PUMAS_RETURN_INTERNAL_ERROR,
                     "could not copy the tables to the device");
@@ -434,6 +495,10 @@ extern "C" enum pumas_return pumas_gpu_physics_upload_memory(
                 ph->step = (const double *)((const uint8_t *)device +
                     step_offset);
                 ph->n_step = (uint32_t)step.size();
+                ph->rows[0] = (const double *)((const uint8_t *)device +
+                    rows_offset);
+                ph->rows[1] = ph->rows[0] + n_rows;
+                ph->n_rows = (uint32_t)n_rows;
 
                 /* In the FP32-bulk copy, K..K_dX (the first four stepped
                  * columns) and a_max, b_max (the last two) follow the
@@ -759,6 +824,7 @@ struct KernelArgs {
         FloatTables ft;
         LdsTables ftl;          /* ft in the stepping kernel's LDS copy */
         LdsStepTables stl;      /* FP64 step tables in the LDS copy */
+        LdsRowTables rowl;      /* or the row tables, in the lean kernels' */
         /* The LDS copy of the stepping kernel: up to three pieces, each
          * `n4` 16 B words from `src` to LDS word `dst`. */
         struct {
@@ -1133,19 +1199,23 @@ __global__ void __launch_bounds__(512, 2) k_step(KernelArgs args, int parity)
 {
         KERNEL_ARGS(args);
         /* With LDS, the tables of the step lookups in the working precision
-         * are read from a copy in LDS: the FP32 mirrors (FP32-bulk) or the
-         * packed FP64 step tables. */
+         * are read from a copy in LDS: the FP32 mirrors (FP32-bulk), the
+         * packed FP64 step tables, or the row tables (lean FP64 kernels). */
         using FT = typename std::conditional<LDS && F32, LdsTables,
             FloatTables>::type;
-        using ST = typename std::conditional<LDS, LdsStepTables,
-            PhysicsView>::type;
+        constexpr bool ROWS = LEAN && !F32; /* as EngineT::ROWS */
+        using ST = typename std::conditional<ROWS, LdsRowTables,
+            typename std::conditional<LDS, LdsStepTables,
+                PhysicsView>::type>::type;
         const FT * ft;
         const ST * st;
         if constexpr (LDS && F32)
                 ft = &a.ftl;
         else
                 ft = &a.ft;
-        if constexpr (LDS)
+        if constexpr (ROWS)
+                st = &a.rowl;
+        else if constexpr (LDS)
                 st = &a.stl;
         else
                 st = &a.p;
@@ -1426,20 +1496,25 @@ struct Launch {
  * instead of 200. */
 using StepKernel = void (*)(KernelArgs, int);
 
+/* The energy loss modes with lean kernels, in launches without a recorder. */
+bool lean_launch(const KernelArgs & a)
+{
+        return (a.rec.frames == nullptr) && (a.c.energy_loss >= MODE_CSDA) &&
+            (a.c.energy_loss <= MODE_STRAGGLED);
+}
+
 template <bool F32>
 StepKernel step_kernel(const KernelArgs & a, bool lds)
 {
         if (!lds) return k_step<F32, false, false, SCHEME_ANY>;
-        if (a.rec.frames) return k_step<F32, true, false, SCHEME_ANY>;
+        if (!lean_launch(a)) return k_step<F32, true, false, SCHEME_ANY>;
         switch (a.c.energy_loss) {
         case MODE_STRAGGLED:
                 return k_step<F32, true, true, MODE_STRAGGLED>;
         case MODE_MIXED:
                 return k_step<F32, true, true, MODE_MIXED>;
-        case MODE_CSDA:
-                return k_step<F32, true, true, MODE_CSDA>;
         default:
-                return k_step<F32, true, false, SCHEME_ANY>;
+                return k_step<F32, true, true, MODE_CSDA>;
         }
 }
 
@@ -1474,12 +1549,14 @@ enum pumas_return allow_lds(StepKernel kernel, int bytes)
 }
 
 /* Bytes of the LDS copy of the step tables in the stepping kernel, or 0
- * when `per_cu` copies do not fit in the LDS of a CU. */
+ * when `per_cu` copies do not fit in the LDS of a CU; sets the pieces of the
+ * copy. Row tables are smaller than the step tables (they hold one energy
+ * loss scheme), which decide. */
 enum pumas_return lds_tables_size(const pumas_gpu_physics * physics,
-    const KernelArgs & a, int device, int per_cu, bool f32, unsigned * bytes)
+    KernelArgs & a, int device, int per_cu, bool f32, unsigned * bytes)
 {
         *bytes = 0;
-        const size_t need = f32 ?
+        size_t need = f32 ?
             (size_t)physics->n_floats * sizeof(float) +
                 (size_t)(physics->range_head + physics->n_step -
                     physics->range_tail_at) * sizeof(double) :
@@ -1491,6 +1568,16 @@ enum pumas_return lds_tables_size(const pumas_gpu_physics * physics,
             hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, device));
         if ((need > (size_t)per_block) || (need * per_cu > (size_t)per_sm))
                 return PUMAS_RETURN_SUCCESS;
+        if (!f32 && lean_launch(a)) {
+                const int scheme = (a.c.energy_loss == MODE_CSDA) ? 0 : 1;
+                need = physics->n_rows * sizeof(double);
+                a.lds_piece[0] = { (const float4 *)physics->rows[scheme], 0,
+                        physics->n_rows / 2 };
+                a.n_lds_pieces = 1;
+                a.rowl.n_energies = physics->view.n_energies;
+                a.rowl.n_materials = physics->view.n_materials;
+                a.rowl.mass = physics->view.mass;
+        }
         if (need > 65536) {
                 const enum pumas_return rc = allow_lds(f32 ?
                         step_kernel<true>(a, true) :
