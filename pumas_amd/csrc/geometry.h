@@ -65,6 +65,19 @@ struct pg_geometry {
         double z_top;
 };
 
+/* A value of the geometry's own arrays at an index that is the same for every
+ * lane of a wavefront: a scalar load on the device (the geometry is not
+ * written while a kernel runs). */
+GEO_FN double geo_uniform(const double * p, int i)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+        typedef const __attribute__((address_space(4))) double geo_cdouble;
+        return ((geo_cdouble *)p)[i];
+#else
+        return p[i];
+#endif
+}
+
 /* Distance along a line to leave [lo, hi) on one axis, or GEO_STEP_FREE. */
 GEO_FN double geo_exit_distance(double x, double u, double lo, double hi)
 {
@@ -141,14 +154,24 @@ GEO_FN int geo_locate(const struct pg_geometry * g, const double * pos,
                 return g->step_type;
 
         case GEO_SLABS: {
+                /* The boundaries ascend, so at most one layer holds z: every
+                 * boundary is read, by scalar loads that do not wait on a
+                 * comparison. (Searched until found, by vector loads one
+                 * after the other, the two locations of a step took a tenth
+                 * of a lone history's time.) */
                 const double z = pos[2];
                 int k = -1;
                 int i;
+                double lo = 0., hi = 0.;
+                double below = geo_uniform(g->z, 0);
                 for (i = 0; i < g->n_layers; i++) {
-                        if ((z >= g->z[i]) && (z < g->z[i + 1])) {
+                        const double above = geo_uniform(g->z, i + 1);
+                        if ((z >= below) && (z < above)) {
                                 k = i;
-                                break;
+                                lo = below;
+                                hi = above;
                         }
+                        below = above;
                 }
                 *medium = k;
                 if (step != 0) {
@@ -156,7 +179,7 @@ GEO_FN int geo_locate(const struct pg_geometry * g, const double * pos,
                                 *step = -1.;
                         } else {
                                 double s = geo_exit_distance(
-                                    z, sgn * dir[2], g->z[k], g->z[k + 1]);
+                                    z, sgn * dir[2], lo, hi);
                                 if (g->step_type == GEO_STEP_RAW)
                                         s += GEO_STEP_EPSILON;
                                 *step = s;
