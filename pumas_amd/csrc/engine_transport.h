@@ -350,6 +350,17 @@ struct EngineT {
                 }
         }
 
+        /* The energy loss at the kinetic energy of an event. */
+        PG_FN double event_energy_loss(Track & t, int scheme, int material) const
+        {
+                if constexpr (ROWS)
+                        return bulk_energy_loss(t, scheme, material,
+                            locate(t, material, t.energy));
+                else
+                        return cel_energy_loss(
+                            p, t.ix, scheme, material, t.energy);
+        }
+
         /* cel_kinetic_energy (src/pumas.c:3758-3784) of the step tables. */
         PG_FN double bulk_kinetic_energy(Track & t, int scheme, int material,
             double grammage) const
@@ -2154,9 +2165,7 @@ struct EngineT {
                         Xf = cel_grammage(
                             p, t.ix, scheme, w.material, t.energy);
                 if ((scheme >= MODE_CSDA) && (c.direction == MODE_BACKWARD))
-                        w.dei = 1. /
-                            cel_energy_loss(
-                                p, t.ix, scheme, w.material, t.energy);
+                        w.dei = 1. / event_energy_loss(t, scheme, w.material);
                 transport_limit(t, w.material, Xi, Xf, &w.grammage_max);
                 if (t.step_event)
                         walker_finish(w);
@@ -2221,8 +2230,7 @@ struct EngineT {
                             lm::exp(-fabs(t.time - w.ti) / p.ctau) :
                             1.;
                         t.weight = (LEAN ? t.weight : w.wi) * wt * w.dei *
-                            cel_energy_loss(p, t.ix, scheme, w.material,
-                                t.energy);
+                            event_energy_loss(t, scheme, w.material);
                 } else if (c.decay == MODE_WEIGHTED) {
                         t.weight = (LEAN ? t.weight : w.wi) *
                             lm::exp(-fabs(t.time - w.ti) / p.ctau);
