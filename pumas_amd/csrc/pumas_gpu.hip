@@ -97,6 +97,28 @@ void pg_clear_error(void) { g_error[0] = '\0'; }
 
 extern "C" const char * pumas_gpu_error_message(void) { return g_error; }
 
+/* Freed with its thread. Copies into pageable memory are staged by the
+ * runtime, with a wait of their own. */
+void * pg_pinned(size_t bytes)
+{
+        struct Buffer {
+                void * p = nullptr;
+                ~Buffer()
+                {
+                        if (p) (void)hipHostFree(p);
+                }
+        };
+        static thread_local Buffer buffer;
+        if (bytes > PG_PINNED_BYTES) return nullptr;
+        if ((buffer.p == nullptr) &&
+            (hipHostMalloc(&buffer.p, PG_PINNED_BYTES,
+                 hipHostMallocPortable) != hipSuccess)) {
+                (void)hipGetLastError();
+                buffer.p = nullptr;
+        }
+        return buffer.p;
+}
+
 extern "C" const char * pumas_gpu_version(void) { return "pumas_hip 0.1.0"; }
 
 extern "C" void pumas_gpu_context_default(struct pumas_gpu_context * context)
@@ -1485,6 +1507,7 @@ struct Launch {
         hipStream_t stream;
         hipEvent_t * marks; /* [2 * rounds_per_check] or NULL */
         hipEvent_t * init_marks; /* [2], around the entry kernel, or NULL */
+        hipEvent_t end_mark; /* after the last kernel, or NULL */
         bool closed; /* every history takes the closed form CSDA */
 };
 
@@ -1677,7 +1700,10 @@ enum pumas_return transport_chunk(const KernelArgs & a0, size_t base,
         a.q_del = reinterpret_cast<uint32_t *>(q + 2 * b_queue);
 
         enum pumas_return rc = PUMAS_RETURN_SUCCESS;
-        unsigned long long host[C_COUNT];
+        unsigned long long stack[C_COUNT];
+        void * const pinned = fixed ? nullptr : pg_pinned(sizeof(stack));
+        unsigned long long * const host =
+            pinned ? static_cast<unsigned long long *>(pinned) : stack;
         hipLaunchKernelGGL(zero_counters, dim3(1), dim3(64), 0, stream,
             a.counters, C_COUNT);
         const unsigned blocks = (unsigned)((m + INIT_BLOCK - 1) / INIT_BLOCK);
@@ -1698,12 +1724,17 @@ enum pumas_return transport_chunk(const KernelArgs & a0, size_t base,
         if (hipGetLastError() != hipSuccess)
                 return pg_fail(PUMAS_RETURN_VALUE_ERROR,
                     "transport kernel launch failed");
+        /* A batch that needs one round (its DELs run in the wavefronts):
+         * the stepping kernel alone, launched without waiting for the entry
+         * kernel's count of the histories to step. */
+        const bool single = !L.closed && ((L.tail_del > 0) ||
+            ((L.tail_del == 0) && (m <= a.wave_del_max)));
         /* The sequence of rounds between two checks is captured once in a
          * HIP graph and replayed (an even number of rounds, so that every
          * replay starts on step queue 0): one launch per check instead of
          * three per round. Counters are cleared by kernels, not memset
          * nodes. */
-        if (L.graph) {
+        if (L.graph && !L.closed && !single) {
                 hipGraph_t graph = nullptr;
                 HIP_TRY(hipStreamBeginCapture(
                     stream, hipStreamCaptureModeThreadLocal));
@@ -1726,12 +1757,25 @@ enum pumas_return transport_chunk(const KernelArgs & a0, size_t base,
         }
         int parity = 0, launched = 0;
         bool init_timed = false;
+        if (single) {
+                if (L.marks) HIP_TRY(hipEventRecord(L.marks[0], stream));
+                if (f32)
+                        launch_step<true>(a, 0, L);
+                else
+                        launch_step<false>(a, 0, L);
+                if (L.marks) HIP_TRY(hipEventRecord(L.marks[1], stream));
+                HIP_TRY(hipGetLastError());
+                if (stats) stats->rounds += 1;
+                launched = 1;
+                parity = 1;
+        }
         for (;;) {
-                HIP_TRY(hipMemcpyAsync(host, a.counters, sizeof(host),
-                    hipMemcpyDeviceToHost, stream));
+                /* The end of the call's work, unless more rounds follow. */
+                if (L.end_mark) HIP_TRY(hipEventRecord(L.end_mark, stream));
+                HIP_TRY(hipMemcpyAsync(host, a.counters,
+                    C_COUNT * sizeof(*host), hipMemcpyDeviceToHost, stream));
                 HIP_TRY(hipStreamSynchronize(stream));
-                if (L.init_marks && stats && (parity == 0) &&
-                    (launched == 0) && !init_timed) {
+                if (L.init_marks && stats && !init_timed) {
                         float ms = 0.f;
                         HIP_TRY(hipEventElapsedTime(&ms, L.init_marks[0],
                             L.init_marks[1]));
@@ -1948,13 +1992,20 @@ static enum pumas_return transport_impl(const pumas_gpu_physics * physics,
                     physics, a, device, per_cu, f32, &lds_bytes);
                 if (rc != PUMAS_RETURN_SUCCESS) return rc;
         }
+        /* Every history takes the closed form CSDA when the geometry has
+         * no step limits (a uniform infinite medium), the energy loss is
+         * CSDA and scattering is disabled (src/pumas.c:3200-3230). */
+        const bool closed = (geometry->view.kind == GEO_INFINITE) &&
+            (geometry->view.locals == nullptr) &&
+            (context->mode.energy_loss == PUMAS_MODE_CSDA) &&
+            (context->mode.scattering == PUMAS_MODE_DISABLED);
         unsigned long long total_steps = 0, error = 0;
         /* The legacy NULL stream cannot be captured. */
         const bool graph = !(options && options->eager) &&
             (stream != nullptr) && !fixed;
         if (stats) {
                 memset(stats, 0x0, sizeof(*stats));
-                if (!graph && !fixed) {
+                if (!graph && !fixed && !closed) {
                         ev.marks.resize(2 * rounds_per_check, nullptr);
                         for (auto & e : ev.marks)
                                 HIP_TRY(hipEventCreate(&e));
@@ -1968,17 +2019,11 @@ static enum pumas_return transport_impl(const pumas_gpu_physics * physics,
                 return pg_fail(PUMAS_RETURN_VALUE_ERROR,
                     "lanes_per_wave must be at most 64 (got %d)",
                     lanes_per_wave);
-        /* Every history takes the closed form CSDA when the geometry has
-         * no step limits (a uniform infinite medium), the energy loss is
-         * CSDA and scattering is disabled (src/pumas.c:3200-3230). */
-        const bool closed = (geometry->view.kind == GEO_INFINITE) &&
-            (geometry->view.locals == nullptr) &&
-            (context->mode.energy_loss == PUMAS_MODE_CSDA) &&
-            (context->mode.scattering == PUMAS_MODE_DISABLED);
         const Launch L = { n_cu, block, per_cu, rounds_per_check, graph,
                 tail_del, lanes_per_wave, lds_bytes, 0, 0, stream,
-                (stats && !graph && !fixed) ? ev.marks.data() : nullptr,
-                (stats && !fixed) ? ev.init : nullptr, closed };
+                ev.marks.empty() ? nullptr : ev.marks.data(),
+                (stats && !fixed) ? ev.init : nullptr,
+                (stats && !fixed) ? ev.e1 : nullptr, closed };
         const size_t chunk = closed ? MAX_CLOSED_CHUNK : MAX_CHUNK;
         for (size_t base = 0; base < n; base += chunk) {
                 const size_t m = (n - base < chunk) ? n - base : chunk;
@@ -1986,11 +2031,13 @@ static enum pumas_return transport_impl(const pumas_gpu_physics * physics,
                     a, base, m, f32, L, &total_steps, &error, stats, fixed);
                 if (rc != PUMAS_RETURN_SUCCESS) break;
         }
-        if (stats && !fixed) HIP_TRY(hipEventRecord(ev.e1, stream));
-        HIP_TRY(hipStreamSynchronize(stream));
+        /* Every chunk has waited for its last kernel; an error ended the call
+         * between two of its launches. */
+        if (rc != PUMAS_RETURN_SUCCESS) HIP_TRY(hipStreamSynchronize(stream));
         if (stats) {
                 float ms = 0.f;
-                if (!fixed) HIP_TRY(hipEventElapsedTime(&ms, ev.e0, ev.e1));
+                if (!fixed && (n > 0) && (rc == PUMAS_RETURN_SUCCESS))
+                        HIP_TRY(hipEventElapsedTime(&ms, ev.e0, ev.e1));
                 stats->steps = total_steps;
                 stats->histories = n;
                 stats->kernel_ms = ms;

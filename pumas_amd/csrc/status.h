@@ -18,6 +18,13 @@ void pg_clear_error(void);
  * record and queue slots). */
 size_t pg_bytes_per_history(void);
 
+/* Pinned host memory of the calling thread for the small results that a call
+ * copies back and waits for (counters, sums): PG_PINNED_BYTES, kept until the
+ * thread ends. NULL for a larger request, or when there is none (the caller
+ * then uses its own memory). */
+#define PG_PINNED_BYTES 16384
+void * pg_pinned(size_t bytes);
+
 #define HIP_TRY(expr)                                                          \
         do {                                                                   \
                 hipError_t e_ = (expr);                                        \

@@ -315,20 +315,29 @@ extern "C" enum pumas_return pumas_gpu_tally(const struct pumas_state * states,
         hipLaunchKernelGGL(k_tally_reduce, dim3(a.n_out), dim3(TALLY_BLOCK), 0,
             stream, partial, grid, out);
         HIP_TRY(hipGetLastError());
-        std::vector<double> host(a.n_out);
-        HIP_TRY(hipMemcpyAsync(host.data(), out, a.n_out * sizeof(double),
-            hipMemcpyDeviceToHost, stream));
+        static_assert((3 + 4 * PUMAS_GPU_TALLY_MAX_BINS) * sizeof(double) <=
+                PG_PINNED_BYTES, "a tally fits in the pinned buffer");
+        const size_t out_bytes = a.n_out * sizeof(double);
+        std::vector<double> own;
+        double * host = static_cast<double *>(pg_pinned(out_bytes));
+        if (host == nullptr) {
+                own.resize(a.n_out);
+                host = own.data();
+        }
+        const hipError_t copied = hipMemcpyAsync(
+            host, out, out_bytes, hipMemcpyDeviceToHost, stream);
         HIP_TRY(hipFreeAsync(partial, stream));
+        HIP_TRY(copied);
         HIP_TRY(hipStreamSynchronize(stream));
 
         result->sum = host[0];
         result->sum2 = host[1];
         result->count = (uint64_t)host[2];
         if (result->energy)
-                memcpy(result->energy, host.data() + 3,
+                memcpy(result->energy, host + 3,
                     2 * a.n_energy * sizeof(double));
         if (result->cos_theta)
-                memcpy(result->cos_theta, host.data() + 3 + 2 * a.n_energy,
+                memcpy(result->cos_theta, host + 3 + 2 * a.n_energy,
                     2 * a.n_cos * sizeof(double));
         return PUMAS_RETURN_SUCCESS;
 }
