@@ -362,22 +362,23 @@ extern "C" enum pumas_return pumas_gpu_physics_upload_memory(
         const size_t total = rows_offset + rows.size() * sizeof(double);
         void * device = nullptr;
         HIP_TRY(hipMalloc(&device, total));
+        /* The derived sections in one copy. */
+        std::vector<uint8_t> derived(total - extra_offset, 0);
+        auto place = [&](size_t offset, const void * src, size_t bytes) {
+                if (bytes > 0)
+                        memcpy(derived.data() + (offset - extra_offset), src,
+                            bytes);
+        };
+        place(extra_offset, component0.data(),
+            component0.size() * sizeof(int32_t));
+        place(float_offset, floats.data(), floats.size() * sizeof(float));
+        place(step_offset, step.data(), step.size() * sizeof(double));
+        place(coarse_offset, coarse.data(), coarse.size() * sizeof(int16_t));
+        place(rows_offset, rows.data(), rows.size() * sizeof(double));
         hipError_t e1 = hipMemcpy(device, image, size, hipMemcpyHostToDevice);
         hipError_t e2 = hipMemcpy((uint8_t *)device + extra_offset,
-            component0.data(), component0.size() * sizeof(int32_t),
-            hipMemcpyHostToDevice);
-        hipError_t e3 = hipMemcpy((uint8_t *)device + float_offset,
-            floats.data(), floats.size() * sizeof(float),
-            hipMemcpyHostToDevice);
-        hipError_t e4 = hipMemcpy((uint8_t *)device + step_offset,
-            step.data(), step.size() * sizeof(double), hipMemcpyHostToDevice);
-        hipError_t e5 = coarse.empty() ? hipSuccess :
-            hipMemcpy((uint8_t *)device + coarse_offset, coarse.data(),
-                coarse.size() * sizeof(int16_t), hipMemcpyHostToDevice);
-        hipError_t e6 = hipMemcpy((uint8_t *)device + rows_offset, rows.data(),
-            rows.size() * sizeof(double), hipMemcpyHostToDevice);
-        if ((e1 != hipSuccess) || (e2 != hipSuccess) || (e3 != hipSuccess) ||
-            (e4 != hipSuccess) || (e5 != hipSuccess) || (e6 != hipSuccess)) {
+            derived.data(), derived.size(), hipMemcpyHostToDevice);
+        if ((e1 != hipSuccess) || (e2 != hipSuccess)) {
                 (void)hipFree(device);
                 return pg_fail(PUMAS_RETURN_INTERNAL_ERROR,
                     "could not copy the tables to the device");
