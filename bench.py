@@ -591,7 +591,7 @@ def main():
                 "bandwidth bound: the stepping kernel keeps a history in "
                 "registers between DEL vertices (a few B of HBM traffic per "
                 "step measured) and is bound by VALU issue over divergent "
-                "lanes (VALUBusy ~66 %, VALUUtilization ~35 %); the closed "
+                "lanes (VALUBusy ~72 %, VALUUtilization ~38 %); the closed "
                 "form entry kernel moves exactly its 208 B per history and "
                 "is bound by the latency of its dependent table lookups, all "
                 "L2 hits (VALUBusy ~32 %); profiles/ holds the counters"),
