@@ -12,6 +12,7 @@ import tempfile
 
 import numpy as np
 
+import restatement
 from pumas_amd import _abi
 from pumas_amd._abi import STATE_DTYPE
 
@@ -197,7 +198,12 @@ LIBRARY_FLUX = os.path.join(HERE, "_ref", "libflux_ref.so")
 
 def flux(kind, cos_theta, kinetic, charge):
     """The reference's example flux models (examples/pumas/flux.c),
-    kind 1 = flux_gaisser, 2 = flux_gccly, evaluated element-wise."""
+    kind 1 = flux_gaisser, 2 = flux_gccly, evaluated element-wise; their
+    numpy restatement where the reference is not built."""
+    if not os.path.exists(LIBRARY_FLUX):
+        model = {1: restatement.flux_gaisser, 2: restatement.flux_gccly}[kind]
+        return model(*(np.asarray(x, np.float64)
+                       for x in (cos_theta, kinetic, charge)))
     if "flux" not in _libs:
         lib = ctypes.CDLL(LIBRARY_FLUX)
         lib.ref_flux_batch.argtypes = [ctypes.c_int, ctypes.c_size_t] + \

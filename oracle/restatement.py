@@ -232,3 +232,33 @@ def transport_csda(tb, states, material, density, backward, limit_distance,
     path = -distance if backward else distance
     s["position"] += path[:, None] * s["direction"]
     return s, event
+
+
+# ---------------------------------------------------------------------------
+# Sea level flux models of the reference's examples (examples/pumas/flux.c).
+# ---------------------------------------------------------------------------
+def _charge_fraction(charge):
+    """Fraction of the flux with the muon's charge, for a charge ratio of
+    1.2766; 1 for a null charge (flux.c:39-52)."""
+    r = 1.2766
+    return np.where(charge < 0, 1 / (1 + r), np.where(charge > 0, r / (1 + r),
+                                                      1.0))
+
+
+def flux_gaisser(cos_theta, kinetic, charge):
+    """Gaisser's parameterisation, per m^2 s sr GeV (flux.c:57-65)."""
+    e = kinetic + 0.10566
+    ec = 1.1 * e * cos_theta
+    return 1.4e3 * e ** -2.7 * (1 / (1 + ec / 115) + 0.054 / (1 + ec / 850)) * \
+        _charge_fraction(charge)
+
+
+def flux_gccly(cos_theta, kinetic, charge):
+    """Guan et al., with Volkova's cos(theta*) (flux.c:70-89)."""
+    p = (0.102573, -0.068287, 0.958633, 0.0407253, 0.817285)
+    cs2 = (cos_theta ** 2 + p[0] ** 2 + p[1] * cos_theta ** p[2] +
+           p[3] * cos_theta ** p[4]) / (1 + p[0] ** 2 + p[1] + p[3])
+    cs = np.sqrt(np.maximum(cs2, 0))
+    e = kinetic + 0.10566
+    return (1 + 3.64 / (e * cs ** 1.29)) ** -2.7 * \
+        flux_gaisser(cs, kinetic, charge)
