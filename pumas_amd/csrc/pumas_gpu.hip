@@ -16,6 +16,7 @@
 #include "../../include/pumas_gpu.h"
 #include "engine_transport.h"
 #include "ptab.h"
+#include "row_tables.h"
 #include "status.h"
 
 using namespace pg;
@@ -164,7 +165,7 @@ struct pumas_gpu_physics {
         uint32_t range_tail_at; /* a_max..b_max: from here to n_step */
         /* Row tables of the CSDA [0], and of the mixed and straggled [1]
          * energy losses, for the lean FP64 kernels' LDS copy. */
-        const double * rows[2];
+        const double * rows[ROW_SCHEMES];
         uint32_t n_rows;        /* doubles in each (even) */
         int particle;
 };
@@ -229,15 +230,33 @@ extern "C" enum pumas_return pumas_gpu_physics_upload_memory(
         enum pumas_return rc = parse_ptab(image, size, &h, sections);
         if (rc != PUMAS_RETURN_SUCCESS) return rc;
 
-        const int nM = h.imeta[PTAB_N_MATERIALS];
         if (h.imeta[PTAB_MAX_COMPONENTS] > MAX_COMPONENTS)
                 return pg_fail(PUMAS_RETURN_VALUE_ERROR,
                     "materials with more than %d elements are not supported",
                     MAX_COMPONENTS);
 
+        /* Row tables, by energy loss scheme; the first reading of the file's
+         * sizes, which it checks. */
+        const int nM = h.imeta[PTAB_N_MATERIALS];
+        std::vector<double> rows;
+        const char * const bad = pack_row_tables(
+            [&](const char * name) {
+                    const Section * s = find(sections, name);
+                    return ((s == nullptr) || (s->dtype != PTAB_F64)) ?
+                        RowSource { nullptr, 0 } :
+                        RowSource { reinterpret_cast<const double *>(
+                                        image + s->offset),
+                                s->count };
+            },
+            nM, h.imeta[PTAB_N_ENERGIES], rows);
+        if (bad != nullptr)
+                return pg_fail(PUMAS_RETURN_FORMAT_ERROR,
+                    "PTAB section `%s' is missing or short", bad);
+        const size_t n_rows = rows.size() / ROW_SCHEMES;
+
         /* Derived section: first component of each material. */
         const Section * sin = find(sections, "elements_in");
-        if (sin == nullptr)
+        if ((sin == nullptr) || (sin->count < (uint64_t)nM))
                 return pg_fail(PUMAS_RETURN_FORMAT_ERROR, "missing elements_in");
         std::vector<int32_t> component0(nM);
         {
@@ -289,52 +308,6 @@ extern "C" enum pumas_return pumas_gpu_physics_upload_memory(
                     reinterpret_cast<const double *>(image + sec->offset);
                 step.insert(step.end(), src, src + sec->count);
                 while (step.size() % 8) step.push_back(0.);
-        }
-
-        /* Row tables, by energy loss scheme. */
-        const size_t nK = h.imeta[PTAB_N_ENERGIES];
-        const size_t n_rows = (nM * nK * ROW_COLUMNS + 1) / 2 * 2;
-        std::vector<double> rows(2 * n_rows, 0.);
-        {
-                static const struct {
-                        const char * name;
-                        int column;
-                        int schemes; /* 0: none, else its first scheme */
-                } columns[] = { { "X", ROW_X, 1 }, { "X_dK", ROW_X_DK, 1 },
-                        { "K_dX", ROW_K_DX, 1 }, { "dE", ROW_DE, 1 },
-                        { "dE_dK", ROW_DE_DK, 1 }, { "Omega", ROW_OMEGA, 0 },
-                        { "Omega_dK", ROW_OMEGA_DK, 0 }, { "CS", ROW_CS, 0 },
-                        { "CS_dK", ROW_CS_DK, 0 }, { "Mu0", ROW_MU0, 0 },
-                        { "Mu0_dK", ROW_MU0_DK, 0 }, { "Ms1", ROW_MS1, 2 },
-                        { "Ms1_dK", ROW_MS1_DK, 2 }, { "Lb", ROW_LB, 0 },
-                        { "K", ROW_K, -1 } };
-                for (const auto & col : columns) {
-                        const Section * sec = find(sections, col.name);
-                        const size_t tables = (col.schemes < 0) ? 1 :
-                            (size_t)nM * (col.schemes + 1);
-                        if ((sec == nullptr) || (sec->dtype != PTAB_F64) ||
-                            (sec->count < tables * nK))
-                                return pg_fail(PUMAS_RETURN_FORMAT_ERROR,
-                                    "PTAB section `%s' is missing or short",
-                                    col.name);
-                        const double * src = reinterpret_cast<const double *>(
-                            image + sec->offset);
-                        for (int sch = 0; sch < 2; sch++)
-                                for (int m = 0; m < nM; m++) {
-                                        /* Ms1 holds one more scheme first. */
-                                        const size_t table =
-                                            (col.schemes < 0) ? 0 :
-                                            (col.schemes == 0) ? m :
-                                            (size_t)(sch + col.schemes - 1) *
-                                                nM + m;
-                                        for (size_t i = 0; i < nK; i++)
-                                                rows[sch * n_rows +
-                                                    (m * nK + i) *
-                                                        ROW_COLUMNS +
-                                                    col.column] =
-                                                    src[table * nK + i];
-                                }
-                }
         }
 
         /* Coarse index of the kinetic energy grid (k_index_fast). */

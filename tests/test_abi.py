@@ -164,3 +164,28 @@ def test_c_caller_compiles_against_reference_header():
                            os.path.join(REPO, "tests", "kernels"),
                            "../_build/abi_check"])
     assert os.access(exe, os.X_OK)
+
+
+@pytest.mark.parametrize("slot,value", [
+    (0, 1 << 30), (0, -1), (0, 0), (0, 1),  # energies
+    (1, 1 << 30), (1, -1), (1, 0)])         # materials
+def test_upload_refuses_sizes_beyond_the_columns(slot, value):
+    """Sizes in the header that the file's columns do not hold are a format
+    error of the C call, not an exception through it. In a process of its own:
+    an exception would end it."""
+    code = f"""
+import ctypes, struct
+import pumas_amd as pa
+data = bytearray(open(pa.physics_path("standard_c005"), "rb").read())
+struct.pack_into("<i", data, 16 + 4 * {slot}, {value})
+h = ctypes.c_void_p()
+buf = (ctypes.c_char * len(data)).from_buffer(data)
+rc = pa.library().pumas_gpu_physics_upload_memory(buf, len(data),
+                                                  ctypes.byref(h))
+assert rc == pa.Return.FORMAT_ERROR, rc
+assert not h.value
+"""
+    import subprocess
+    import sys
+    subprocess.run([sys.executable, "-c", code], check=True, cwd=REPO,
+                   timeout=120)
