@@ -948,14 +948,17 @@ struct RowTables {
                         if (x < rows[first + c]) return -1;
                         if (x >= rows[first + last * ROW_COLUMNS + c])
                                 return last;
+                        /* A NaN ends in the last row, not in the first one,
+                         * which the multiple scattering does not interpolate.
+                         */
                         i = 0;
                         int j = last;
                         do {
                                 const int k = (i + j) / 2;
-                                if (x >= rows[first + k * ROW_COLUMNS + c])
-                                        i = k;
-                                else
+                                if (x < rows[first + k * ROW_COLUMNS + c])
                                         j = k;
+                                else
+                                        i = k;
                         } while (j - i >= 2);
                         x0 = rows[first + i * ROW_COLUMNS + c];
                         x1 = rows[first + (i + 1) * ROW_COLUMNS + c];

@@ -13,6 +13,7 @@
 #include "../include/pumas_gpu.h"
 #include "engine_transport.h"
 #include "ptab.h"
+#include "row_tables.h"
 
 using namespace pg;
 
@@ -217,4 +218,72 @@ extern "C" void host_cel(int which, int scheme, int material, const double *x,
         default: out[i] = 0.;
         }
     }
+}
+
+/* The per step lookups of the engine on the loaded tables, by the general
+ * engine (lean 0) or by the one compiled for an energy loss scheme, on the row
+ * tables packed as for the device (lean 1): 0 grammage, 1 energy loss,
+ * 2 straggling, 3 DEL cross section, 4 EHS length, 5 and 6 the multiple
+ * scattering's mu0 and inverse path, at a kinetic energy; 7 the kinetic energy
+ * of a grammage; 8 the energy loss of an event. `guess` is the first guess of
+ * the row. Returns 0, or -1 when the rows cannot be packed. */
+template <class E>
+static void lookups(const E &eng, int which, int scheme, int material,
+    const double *x, const int *guess, double *out, int64_t n) {
+    for (int64_t i = 0; i < n; i++) {
+        Track t; memset(&t, 0, sizeof(t));
+        t.ix.k[0] = t.ix.k[1] = t.ix.x[0] = t.ix.x[1] = guess[i];
+        t.energy = x[i];
+        const Located l = eng.locate(t, material, x[i]);
+        double mu0 = 0., invlb1 = 0.;
+        switch (which) {
+        case 0: out[i] = eng.bulk_grammage(t, scheme, material, l); break;
+        case 1: out[i] = eng.bulk_energy_loss(t, scheme, material, l); break;
+        case 2: out[i] = eng.bulk_straggling(t, material, l); break;
+        case 3: out[i] = eng.bulk_del_cross_section(t, material, l); break;
+        case 4: out[i] = eng.bulk_ehs_length(t, material, l); break;
+        case 5: case 6:
+            eng.bulk_msc(t, scheme, material, l, &mu0, &invlb1);
+            out[i] = (which == 5) ? mu0 : invlb1; break;
+        case 7: out[i] = eng.bulk_kinetic_energy(t, scheme, material, x[i]); break;
+        default: out[i] = eng.event_energy_loss(t, scheme, material);
+        }
+    }
+}
+
+template <int SCHEME>
+static void lean_lookups(const RowTables<const double *> &rows, const Config &c,
+    int which, int material, const double *x, const int *guess, double *out,
+    int64_t n) {
+    static FloatTables ft; static pg_geometry g;
+    const EngineT<false, FloatTables, RowTables<const double *>, true, SCHEME>
+        eng = {g_view, g_mv, c, g, ft, rows, g_rec};
+    lookups(eng, which, SCHEME, material, x, guess, out, n);
+}
+
+extern "C" int host_lookups(int lean, int which, int scheme, int material,
+    const double *x, const int *guess, double *out, int64_t n) {
+    Config c; memset(&c, 0, sizeof(c)); c.energy_loss = scheme;
+    static FloatTables ft; static pg_geometry g;
+    if (!lean) {
+        Engine eng = {g_view, g_mv, c, g, ft, g_view, g_rec};
+        lookups(eng, which, scheme, material, x, guess, out, n);
+        return 0;
+    }
+    std::vector<double> packed;
+    const ptab_header *h = (const ptab_header *)g_image.data();
+    const ptab_entry *e = (const ptab_entry *)(g_image.data() + sizeof(ptab_header));
+    if (pack_row_tables([&](const char *name) {
+            for (uint32_t i = 0; i < h->n_entries; i++)
+                if (!strncmp(e[i].name, name, PTAB_NAME_LEN))
+                    return RowSource{(const double *)(g_image.data() + e[i].offset), e[i].count};
+            return RowSource{nullptr, 0};
+        }, g_view.n_materials, g_view.n_energies, packed)) return -1;
+    RowTables<const double *> rows; memset(&rows, 0, sizeof(rows));
+    rows.n_energies = g_view.n_energies;
+    rows.rows = packed.data() + ((scheme == MODE_CSDA) ? 0 : packed.size() / ROW_SCHEMES);
+    if (scheme == MODE_CSDA) lean_lookups<MODE_CSDA>(rows, c, which, material, x, guess, out, n);
+    else if (scheme == MODE_MIXED) lean_lookups<MODE_MIXED>(rows, c, which, material, x, guess, out, n);
+    else lean_lookups<MODE_STRAGGLED>(rows, c, which, material, x, guess, out, n);
+    return 0;
 }
