@@ -2006,8 +2006,10 @@ static enum pumas_return transport_impl(const pumas_gpu_physics * physics,
                 if (rc != PUMAS_RETURN_SUCCESS) break;
         }
         /* Every chunk has waited for its last kernel; an error ended the call
-         * between two of its launches. */
-        if (rc != PUMAS_RETURN_SUCCESS) HIP_TRY(hipStreamSynchronize(stream));
+         * between two of its launches, and an empty batch has no chunk: the
+         * call returns with the stream's work done all the same. */
+        if ((rc != PUMAS_RETURN_SUCCESS) || (n == 0))
+                HIP_TRY(hipStreamSynchronize(stream));
         if (stats) {
                 float ms = 0.f;
                 if (!fixed && (n > 0) && (rc == PUMAS_RETURN_SUCCESS))
