@@ -98,19 +98,41 @@ void pg_clear_error(void) { g_error[0] = '\0'; }
 
 extern "C" const char * pumas_gpu_error_message(void) { return g_error; }
 
-/* Freed with its thread. Copies into pageable memory are staged by the
- * runtime, with a wait of their own. */
+/* A thread's buffer is its own until it ends, and then the next thread's: a
+ * program with a thread per call would else allocate and free one in every call.
+ * Up to PINNED_IDLE of them wait, the others are freed. The list is never
+ * destroyed, as threads may end after static objects. Copies into pageable
+ * memory are staged by the runtime, with a wait of their own. */
 void * pg_pinned(size_t bytes)
 {
+        constexpr int PINNED_IDLE = 16;
+        struct Idle {
+                std::mutex mu;
+                void * p[PINNED_IDLE];
+                int n = 0;
+        };
+        static Idle & idle = *new Idle;
         struct Buffer {
                 void * p = nullptr;
                 ~Buffer()
                 {
-                        if (p) (void)hipHostFree(p);
+                        if (p == nullptr) return;
+                        {
+                                std::lock_guard<std::mutex> lock(idle.mu);
+                                if (idle.n < PINNED_IDLE) {
+                                        idle.p[idle.n++] = p;
+                                        return;
+                                }
+                        }
+                        (void)hipHostFree(p);
                 }
         };
         static thread_local Buffer buffer;
         if (bytes > PG_PINNED_BYTES) return nullptr;
+        if (buffer.p == nullptr) {
+                std::lock_guard<std::mutex> lock(idle.mu);
+                if (idle.n > 0) buffer.p = idle.p[--idle.n];
+        }
         if ((buffer.p == nullptr) &&
             (hipHostMalloc(&buffer.p, PG_PINNED_BYTES,
                  hipHostMallocPortable) != hipSuccess)) {

@@ -21,7 +21,8 @@ size_t pg_bytes_per_history(void);
 /* Pinned host memory of the calling thread for the small results that a call
  * copies back and waits for (counters, sums): PG_PINNED_BYTES, kept until the
  * thread ends. NULL for a larger request, or when there is none (the caller
- * then uses its own memory). */
+ * then uses its own memory). No copy into it may be in flight when a call
+ * returns. */
 #define PG_PINNED_BYTES 16384
 void * pg_pinned(size_t bytes);
 

@@ -326,9 +326,11 @@ extern "C" enum pumas_return pumas_gpu_tally(const struct pumas_state * states,
         }
         const hipError_t copied = hipMemcpyAsync(
             host, out, out_bytes, hipMemcpyDeviceToHost, stream);
-        HIP_TRY(hipFreeAsync(partial, stream));
-        HIP_TRY(copied);
+        const hipError_t freed = hipFreeAsync(partial, stream);
+        /* First, so that no copy into `host` outlasts the call. */
         HIP_TRY(hipStreamSynchronize(stream));
+        HIP_TRY(copied);
+        HIP_TRY(freed);
 
         result->sum = host[0];
         result->sum2 = host[1];
