@@ -199,6 +199,7 @@ struct Rng {
  * Physics tables in device memory (PTAB sections, see ptab.h).
  * ------------------------------------------------------------------------ */
 struct PhysicsView {
+        static constexpr bool by_rows = false;
         int n_energies, n_materials, n_elements, n_components, n_table_dcs;
         int max_components;
         double mass, ctau, cutoff;
@@ -916,6 +917,7 @@ struct Located {
 
 template <class C>
 struct RowTables {
+        static constexpr bool by_rows = true;
         int n_energies, n_materials;
         double mass;
         C rows; /* [material][row][ROW_COLUMNS] */

@@ -152,8 +152,10 @@ static PG_NOINLINE void record_state(const Recorder rec, const Track t,
         f.reserved = 0;
 }
 
-/* SCHEME of an engine that reads the energy loss mode from its Config. */
+/* SCHEME of an engine that reads the energy loss mode from its Config: any
+ * mode, or any but CSDA, mixed and straggled losses. */
 constexpr int SCHEME_ANY = -2;
+constexpr int SCHEME_NONE = -3;
 
 /*
  * The transport engine. With F32 false every operation is the reference's
@@ -205,13 +207,21 @@ struct EngineT {
          * one). */
         PG_FN int loss() const
         {
-                return (SCHEME == SCHEME_ANY) ? c.energy_loss : SCHEME;
+                if constexpr ((SCHEME == SCHEME_ANY) ||
+                    (SCHEME == SCHEME_NONE)) {
+                        const int l = c.energy_loss;
+                        if ((SCHEME == SCHEME_NONE) && (l >= MODE_CSDA) &&
+                            (l <= MODE_STRAGGLED))
+                                __builtin_unreachable();
+                        return l;
+                } else
+                        return SCHEME;
         }
 
         /* Per-step table lookups at a located energy: interpolations of the
-         * row tables in a lean FP64 engine, else the accessors, in the bulk
+         * row tables where `st` holds them, else the accessors, in the bulk
          * precision, at its kinetic energy. */
-        static constexpr bool ROWS = LEAN && !F32;
+        static constexpr bool ROWS = ST::by_rows;
 
         PG_FN Located locate(Track & t, int material, double kinetic) const
         {

@@ -62,6 +62,7 @@ struct LdsDoubles {
  * stopping power and its inverse, straggling, DEL cross section, MSC and
  * EHS parameters), as columns of the LDS copy. */
 struct LdsStepTables {
+        static constexpr bool by_rows = false;
         int n_energies, n_materials;
         double mass;
         LdsDoubles K, X, X_dK, K_dX, dE, dE_dK, Omega, Omega_dK;
@@ -73,7 +74,7 @@ struct LdsStepTables {
         static constexpr bool coarse_index = false;
 };
 
-/* The row tables, the whole LDS copy of the lean FP64 kernels. */
+/* The row tables, the whole LDS copy of the FP64 kernels with energy loss. */
 struct LdsRowColumn {
         PG_FN double operator[](int i) const { return pg_lds_doubles[i]; }
 };
@@ -1217,11 +1218,12 @@ __global__ void __launch_bounds__(512, 2) k_step(KernelArgs args, int parity)
 {
         KERNEL_ARGS(args);
         /* With LDS, the tables of the step lookups in the working precision
-         * are read from a copy in LDS: the FP32 mirrors (FP32-bulk), the
-         * packed FP64 step tables, or the row tables (lean FP64 kernels). */
+         * are read from a copy in LDS: the FP32 mirrors (FP32-bulk), the row
+         * tables (lean FP64 kernels with energy loss) or the packed FP64 step
+         * tables. */
         using FT = typename std::conditional<LDS && F32, LdsTables,
             FloatTables>::type;
-        constexpr bool ROWS = LEAN && !F32; /* as EngineT::ROWS */
+        constexpr bool ROWS = LEAN && LDS && !F32 && (SCHEME >= MODE_CSDA);
         using ST = typename std::conditional<ROWS, LdsRowTables,
             typename std::conditional<LDS, LdsStepTables,
                 PhysicsView>::type>::type;
@@ -1239,6 +1241,10 @@ __global__ void __launch_bounds__(512, 2) k_step(KernelArgs args, int parity)
                 st = &a.p;
         const EngineT<F32, FT, ST, LEAN, SCHEME> eng = { a.p, a.mv, a.c, a.g,
                 *ft, *st, a.rec, a.records };
+        /* The modes with inelastic DELs. The others have no DEL call, and
+         * spill nothing around it (10^6 muons, CSDA: 205 -> 196 ms, FP32 186
+         * -> 181). */
+        constexpr bool DELS = (SCHEME == SCHEME_ANY) || (SCHEME > MODE_CSDA);
         const uint64_t below = lanes_below();
         const uint32_t * in = a.q_step[parity];
         const unsigned long long n_in = a.counters[C_STEP_N0 + parity];
@@ -1302,8 +1308,8 @@ __global__ void __launch_bounds__(512, 2) k_step(KernelArgs args, int parity)
                                             a.states + slot);
                                 steps_acc += w.t.steps;
                         }
-                        const bool to_del = del && !wave_del;
-                        uint64_t dels = __ballot(del && wave_del);
+                        const bool to_del = DELS && del && !wave_del;
+                        uint64_t dels = DELS ? __ballot(del && wave_del) : 0;
                         if (dels) {
                                 const int others = __popcll(
                                     __ballot((w.phase == PHASE_STEP) ||
@@ -1418,9 +1424,11 @@ __global__ void __launch_bounds__(512, 2) k_step(KernelArgs args, int parity)
                                 if (w.phase == PHASE_EHS) eng.walker_ehs(w);
                         }
                 }
-                if (!finished)
-                        del_wave<F32>(
-                            &a, slot, (del_mask >> (threadIdx.x & 63)) & 1);
+                if constexpr (DELS) {
+                        if (!finished)
+                                del_wave<F32>(&a, slot,
+                                    (del_mask >> (threadIdx.x & 63)) & 1);
+                }
         } while (!finished);
         steps_flush(a, steps_acc);
 }
@@ -1507,40 +1515,48 @@ struct Launch {
         bool closed; /* every history takes the closed form CSDA */
 };
 
-/* The stepping kernel of a launch. The lean kernels, compiled for one energy
- * loss mode, serve the launches without a frame recorder whose step tables
- * fit in LDS; the general one the others (recorders, launch shapes with
- * several LDS copies per CU, transport without energy loss). Compiled for any
- * mode, the lean FP64 kernel with in-wavefront DELs spilled 1014 registers
- * instead of 200. */
+/* The stepping kernel of a launch. The lean kernels are compiled for one energy
+ * loss mode; the general one serves the launches with a frame recorder. In the
+ * general kernel, 10^6 muons through the slabs took, without energy loss, 65 ms
+ * (FP32 65) instead of 50 (42), and with the tables in HBM, CSDA, 277 ms (288)
+ * instead of 216 (193). */
 using StepKernel = void (*)(KernelArgs, int);
 
-/* The energy loss modes with lean kernels, in launches without a recorder. */
-bool lean_launch(const KernelArgs & a)
+template <bool F32, bool LDS>
+StepKernel step_kernel(const KernelArgs & a)
 {
-        return (a.rec.frames == nullptr) && (a.c.energy_loss >= MODE_CSDA) &&
+        if (a.rec.frames != nullptr) return k_step<F32, LDS, false, SCHEME_ANY>;
+        switch (a.c.energy_loss) {
+        case MODE_STRAGGLED:
+                return k_step<F32, LDS, true, MODE_STRAGGLED>;
+        case MODE_MIXED:
+                return k_step<F32, LDS, true, MODE_MIXED>;
+        case MODE_CSDA:
+                return k_step<F32, LDS, true, MODE_CSDA>;
+        default:
+                return k_step<F32, LDS, true, SCHEME_NONE>;
+        }
+}
+
+/* Whether that kernel reads the row tables from its LDS copy. */
+bool row_launch(const KernelArgs & a, bool f32)
+{
+        return !f32 && (a.rec.frames == nullptr) &&
+            (a.c.energy_loss >= MODE_CSDA) &&
             (a.c.energy_loss <= MODE_STRAGGLED);
 }
 
-template <bool F32>
-StepKernel step_kernel(const KernelArgs & a, bool lds)
+StepKernel step_kernel(const KernelArgs & a, bool f32, bool lds)
 {
-        if (!lds) return k_step<F32, false, false, SCHEME_ANY>;
-        if (!lean_launch(a)) return k_step<F32, true, false, SCHEME_ANY>;
-        switch (a.c.energy_loss) {
-        case MODE_STRAGGLED:
-                return k_step<F32, true, true, MODE_STRAGGLED>;
-        case MODE_MIXED:
-                return k_step<F32, true, true, MODE_MIXED>;
-        default:
-                return k_step<F32, true, true, MODE_CSDA>;
-        }
+        if (f32) return lds ? step_kernel<true, true>(a) :
+                              step_kernel<true, false>(a);
+        return lds ? step_kernel<false, true>(a) : step_kernel<false, false>(a);
 }
 
 template <bool F32>
 void launch_step(const KernelArgs & a, int parity, const Launch & L)
 {
-        hipLaunchKernelGGL(step_kernel<F32>(a, L.lds_bytes > 0),
+        hipLaunchKernelGGL(step_kernel(a, F32, L.lds_bytes > 0),
             dim3(L.step_grid), dim3(L.block), L.lds_bytes, L.stream, a, parity);
 }
 
@@ -1587,7 +1603,7 @@ enum pumas_return lds_tables_size(const pumas_gpu_physics * physics,
             hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, device));
         if ((need > (size_t)per_block) || (need * per_cu > (size_t)per_sm))
                 return PUMAS_RETURN_SUCCESS;
-        if (!f32 && lean_launch(a)) {
+        if (row_launch(a, f32)) {
                 const int scheme = (a.c.energy_loss == MODE_CSDA) ? 0 : 1;
                 need = physics->n_rows * sizeof(double);
                 a.lds_piece[0] = { (const float4 *)physics->rows[scheme], 0,
@@ -1598,10 +1614,8 @@ enum pumas_return lds_tables_size(const pumas_gpu_physics * physics,
                 a.rowl.mass = physics->view.mass;
         }
         if (need > 65536) {
-                const enum pumas_return rc = allow_lds(f32 ?
-                        step_kernel<true>(a, true) :
-                        step_kernel<false>(a, true),
-                    (int)need);
+                const enum pumas_return rc =
+                    allow_lds(step_kernel(a, f32, true), (int)need);
                 if (rc != PUMAS_RETURN_SUCCESS) return rc;
         }
         *bytes = (unsigned)need;
