@@ -14,72 +14,10 @@
 #include <vector>
 
 #include "../../include/pumas_gpu.h"
-#include "engine_transport.h"
 #include "ptab.h"
 #include "row_tables.h"
+#include "scheduler.h"
 #include "status.h"
-
-using namespace pg;
-
-/* Dynamic LDS of the FP32-bulk stepping kernel: a copy of the single
- * precision tables, made by each block at its start. */
-extern __shared__ float pg_lds_floats[];
-
-/* A table column in that copy, as an offset in floats. Reads compile to LDS
- * loads (ds_read) addressed from the symbol, so the table view holding these
- * offsets stays in the kernel arguments (scalar registers). */
-struct LdsFloats {
-        uint32_t off;
-
-        PG_FN float operator[](int i) const { return pg_lds_floats[off + i]; }
-        PG_FN LdsFloats operator+(int k) const
-        {
-                return LdsFloats{ off + (uint32_t)k };
-        }
-};
-
-using LdsTables = FloatTablesT<LdsFloats>;
-
-/* The same for the FP64 stepping kernel: the tables read by every step. */
-extern __shared__ double pg_lds_doubles[];
-
-struct LdsDoubles {
-        uint32_t off;
-
-        PG_FN double operator[](int i) const { return pg_lds_doubles[off + i]; }
-        PG_FN double operator*() const { return pg_lds_doubles[off]; }
-        PG_FN LdsDoubles operator+(int k) const
-        {
-                return LdsDoubles{ off + (uint32_t)k };
-        }
-        PG_FN bool operator==(const LdsDoubles & o) const
-        {
-                return off == o.off;
-        }
-};
-
-/* The members of PhysicsView that the per-step lookups read (CEL range,
- * stopping power and its inverse, straggling, DEL cross section, MSC and
- * EHS parameters), as columns of the LDS copy. */
-struct LdsStepTables {
-        static constexpr bool by_rows = false;
-        int n_energies, n_materials;
-        double mass;
-        LdsDoubles K, X, X_dK, K_dX, dE, dE_dK, Omega, Omega_dK;
-        LdsDoubles CS, CS_dK, Mu0, Mu0_dK, Ms1, Ms1_dK, Lb, a_max, b_max;
-        const int16_t * k_coarse; /* in HBM, as PhysicsView::k_coarse */
-        int k_bin0, k_nbins;
-        /* The stepping kernel's lookups rarely miss far: no coarse index
-         * code in it. */
-        static constexpr bool coarse_index = false;
-};
-
-/* The row tables, the whole LDS copy of the FP64 kernels with energy loss. */
-struct LdsRowColumn {
-        PG_FN double operator[](int i) const { return pg_lds_doubles[i]; }
-};
-
-using LdsRowTables = RowTables<LdsRowColumn>;
 
 /* ------------------------------------------------------------------------
  * Error reporting.
@@ -799,92 +737,6 @@ extern "C" enum pumas_return pumas_gpu_geometry_create(
         return PUMAS_RETURN_SUCCESS;
 }
 
-/* ------------------------------------------------------------------------
- * Transport kernels: a wavefront scheduler over per-phase queues.
- *
- * A batch runs in rounds. k_init loads every history and runs the entry
- * logic of pumas_context_transport; histories that need stepping get a
- * record (their Walker, in HBM) and a slot in the step queue. Each round
- * then runs two kernels:
- *   k_step  persistent; a lane takes a slot from the step queue and steps
- *           that history in registers, elastic hard scatterings (EHS)
- *           included, until it ends or reaches an inelastic DEL vertex,
- *           then writes it back and appends its slot to the DEL queue (one
- *           atomic per wavefront); free lanes refill by ballot;
- *   k_del   one lane per queued DEL, all lanes on the same sampling code;
- *           the histories go back to the next round's step queue.
- * EHS vertices (~16% of the steps of a muon in rock) are batched inside the
- * stepping wavefront: lanes that reach one wait until enough others do.
- * DEL vertices (~0.2% of the steps at a 5% cutoff) leave the wavefront in the
- * rounds of large batches, and leave the stepping loop in the other rounds:
- * the DEL samplers are the largest code of the path (exact DCS models, polar
- * angles, rejection loops) and would hold the stepping kernel's registers
- * for every step. A history's operations are the reference's, in its
- * order; only the interleaving across histories differs, and the random
- * stream of a history is keyed by its id, so results do not depend on the
- * schedule.
- * ------------------------------------------------------------------------ */
-enum {
-        C_TAKEN = 0, /* step queue entries taken in this round */
-        C_STEPS,     /* Monte Carlo steps of finished histories */
-        C_ERROR,     /* first error code raised by a history */
-        C_STEP_N0,   /* step queue lengths (ping-pong) */
-        C_STEP_N1,
-        C_DEL_N,     /* DEL queue length */
-        C_STATUS,    /* histories ended with HISTORY_STEP_LIMIT, then */
-        C_STATUS_LOOP,   /* HISTORY_LOOP_LIMIT and */
-        C_STATUS_TARGET, /* HISTORY_NO_TARGET */
-        C_COUNT = 12
-};
-
-struct KernelArgs {
-        PhysicsView p;
-        ModelView mv;
-        FloatTables ft;
-        LdsTables ftl;          /* ft in the stepping kernel's LDS copy */
-        LdsStepTables stl;      /* FP64 step tables in the LDS copy */
-        LdsRowTables rowl;      /* or the row tables, in the lean kernels' */
-        /* The LDS copy of the stepping kernel: up to three pieces, each
-         * `n4` 16 B words from `src` to LDS word `dst`. */
-        struct {
-                const float4 * src;
-                uint32_t dst, n4;
-        } lds_piece[3];
-        int n_lds_pieces;
-        Config c;
-        pg_geometry g;
-        struct pumas_state * states;
-        uint64_t n;
-        uint64_t seed;
-        uint64_t first;
-        enum pumas_event * events;
-        int32_t * media;
-        uint32_t * steps;
-        uint32_t * draws;
-        int32_t * rc;
-        int max_steps;
-        int ehs_batch;
-        uint32_t resident_lanes; /* of the stepping launch */
-        uint64_t wave_del_max;   /* histories of a round up to which DELs are
-                                    applied in the wavefronts */
-        int lanes_per_wave;      /* lanes of a wavefront taking histories */
-        int lanes_auto;          /* fewer in the rounds that fit (k_step) */
-        int tail_del;            /* as pumas_gpu_options.tail_del */
-        Recorder rec;
-        unsigned long long * counters;
-        Walker * records;     /* [n] histories in flight */
-        uint32_t * q_step[2]; /* [n] step queues (ping-pong) */
-        uint32_t * q_del;     /* [n] */
-};
-
-/* The arguments are read in place from the kernarg segment (scalar loads of
- * uniform data): naming the by-value parameter's members by reference would
- * make a per-lane scratch copy of it. */
-#define KERNEL_ARGS(args)                                                      \
-        (void)(args);                                                          \
-        const KernelArgs & a =                                                 \
-            *(const KernelArgs *)__builtin_amdgcn_kernarg_segment_ptr()
-
 /* Load history i, whose state is at `s`, into a walker. */
 __device__ __forceinline__ void walker_load(const KernelArgs & a, uint64_t i,
     Walker & w, const struct pumas_state * s)
@@ -913,115 +765,6 @@ __device__ __forceinline__ void walker_load(const KernelArgs & a, uint64_t i,
         t.rng.init(a.seed, a.first + i, STREAM_TRANSPORT, 0);
         t.steps = 0;
         t.max_steps = a.max_steps;
-}
-
-/* Store the end state of history i at `s` and its outputs. `cold` holds the
- * members that a lean engine leaves in the record (`w` itself otherwise). */
-__device__ __forceinline__ void walker_store(const KernelArgs & a, uint64_t i,
-    const Walker & w, const Walker & cold, struct pumas_state * s)
-{
-        const Track & t = w.t;
-        const int rc = cold.rc;
-        s->charge = cold.t.charge;
-        s->energy = t.energy;
-        s->distance = t.distance;
-        s->grammage = t.grammage;
-        s->time = t.time;
-        s->weight = t.weight;
-        s->position[0] = t.pos[0];
-        s->position[1] = t.pos[1];
-        s->position[2] = t.pos[2];
-        s->direction[0] = t.dir[0];
-        s->direction[1] = t.dir[1];
-        s->direction[2] = t.dir[2];
-        s->decayed = cold.t.decayed;
-        if (a.events) a.events[i] = (enum pumas_event)cold.event;
-        if (a.media) {
-                a.media[2 * i] = cold.media0;
-                a.media[2 * i + 1] = cold.end_medium;
-        }
-        if (a.steps) a.steps[i] = t.steps;
-        if (a.draws) a.draws[i] = t.rng.count;
-        if (a.rc) a.rc[i] = rc;
-        if (rc >= HISTORY_STEP_LIMIT)
-                atomicAdd(a.counters + C_STATUS + (rc - HISTORY_STEP_LIMIT),
-                    1ull);
-        else if (rc != RETURN_SUCCESS)
-                atomicCAS(a.counters + C_ERROR, 0ull, (unsigned long long)rc);
-}
-
-/* Write a history back to its record; of a lean engine, only the members
- * that it keeps in registers. */
-template <bool F32, bool LEAN>
-__device__ __forceinline__ void walker_save(Walker * r, const Walker & w)
-{
-        if constexpr (!LEAN) {
-                *r = w;
-                return;
-        }
-        r->t.energy = w.t.energy;
-        r->t.distance = w.t.distance;
-        r->t.grammage = w.t.grammage;
-        r->t.time = w.t.time;
-        r->t.weight = w.t.weight;
-        for (int i = 0; i < 3; i++) {
-                r->t.pos[i] = w.t.pos[i];
-                r->t.dir[i] = w.t.dir[i];
-        }
-        r->t.step_first = w.t.step_first;
-        r->t.step_event = w.t.step_event;
-        r->t.step_foreseen = w.t.step_foreseen;
-        r->t.step_invlb1 = w.t.step_invlb1;
-        r->t.randn_done = w.t.randn_done;
-        r->t.randn_next = w.t.randn_next;
-        r->t.ix = w.t.ix;
-        if constexpr (F32) r->t.fx = w.t.fx;
-        r->t.rng.count = w.t.rng.count;
-        r->t.rng.next_lo = w.t.rng.next_lo;
-        r->t.rng.next_hi = w.t.rng.next_hi;
-        r->t.steps = w.t.steps;
-        r->t.max_steps = w.t.max_steps;
-        r->phase = w.phase;
-        r->medium = w.medium;
-        r->material = w.material;
-        r->straight = w.straight;
-        r->step_index = w.step_index;
-        r->step_max_type = w.step_max_type;
-        r->density = w.density;
-        r->step_max_medium = w.step_max_medium;
-        r->step_max_locals = w.step_max_locals;
-        r->ti = w.ti;
-        r->dei = w.dei;
-        r->grammage_max = w.grammage_max;
-}
-
-__device__ __forceinline__ uint64_t lanes_below()
-{
-        const int lane = threadIdx.x & 63;
-        return (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-}
-
-/* Append `slot` to `queue` for the lanes where `pred` holds: one atomic per
- * wavefront, positions by prefix count. Called by all lanes of the wave. */
-__device__ __forceinline__ void queue_append(unsigned long long * count,
-    uint32_t * queue, bool pred, uint32_t slot)
-{
-        const uint64_t m = __ballot(pred);
-        if (!m) return;
-        const int leader = __ffsll((unsigned long long)m) - 1;
-        unsigned long long base = 0;
-        if ((int)(threadIdx.x & 63) == leader)
-                base = atomicAdd(count, (unsigned long long)__popcll(m));
-        base = __shfl(base, leader, 64);
-        if (pred) queue[base + __popcll(m & lanes_below())] = slot;
-}
-
-/* Sum a per-lane step tally over the wave into the global counter. */
-__device__ __forceinline__ void steps_flush(
-    const KernelArgs & a, unsigned long long acc)
-{
-        for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
-        if ((threadIdx.x & 63) == 0 && acc) atomicAdd(a.counters + C_STEPS, acc);
 }
 
 /* Entry of every history of the batch; one lane per history. The
@@ -1142,297 +885,6 @@ __global__ void k_round(unsigned long long * c, int parity)
         }
 }
 
-/*
- * Schedule of the stepping rounds. Slabs forward FP64, and the same with
- * backward voxels (1 % cutoff, a DEL every 20 steps), 256 CUs x 512 lanes.
- *
- * WAVE_DEL_ROUNDS: a round of at most so many times the resident lanes has its
- * DELs in the wavefronts, so that it ends the batch; a larger one queues them
- * for a kernel that runs 64 of them per wavefront. 1 (and queued until the
- * step queue is exhausted): 2x10^5 muons 147 ms, 10^6 354, 3x10^6 809, voxels
- * 10^6 121; 2: 74, 324, 782, 119; 4: 77, 306, 775, 121; 8: 77, 292, 771, 139.
- * DEL_BATCH, DEL_WAIT: such DELs run when so many lanes, or as many as the
- * others in flight, wait for one, or after so many steps of the others, as
- * one lane's DEL costs the wavefront as much as many lanes'. At once: voxels
- * 5x10^4 35.9 ms, terrain 10^5 62.1; 8, 32: 27.6, 55.7; 24, 48: 26.6, 55.9.
- * HAND_OVER: in a larger round, a wavefront with fewer than so many of 64
- * lanes left, once the step queue is exhausted, puts its histories in the next
- * round's queue, instead of stepping them until the last one ends: 0: 10^6
- * muons 379 ms, voxels 10^6 179, terrain 6x10^5 200; 32: 354, 128, 137; 48:
- * 377, 126, 131. Not before HAND_OVER_AFTER steps, so that every round makes
- * progress.
- * PACK_LANES: a round that fits with more than so many lanes per wavefront, and
- * in half of the wavefronts of each 512 lane block, is put in that half: one
- * wavefront per SIMD with twice the lanes. 30011 muons 48.2 -> 45.2 ms, 60000
- * 53.4 -> 48.6; below it loses: 3000 29.8 -> 32.7, 10000 38.6 -> 40.6.
- */
-constexpr uint64_t WAVE_DEL_ROUNDS = 4;
-constexpr int DEL_BATCH = 24;
-constexpr int DEL_WAIT = 48;
-constexpr int HAND_OVER = 40;
-constexpr int HAND_OVER_AFTER = 32;
-constexpr uint32_t PACK_LANES = 8;
-
-/* The kernel arguments at `args` (the kernarg segment), the same for every
- * lane: in scalar registers, so that their members are scalar loads also in
- * out-of-line code. */
-__device__ __forceinline__ const KernelArgs & uniform_args(
-    const KernelArgs * args)
-{
-        typedef const __attribute__((address_space(4))) KernelArgs cargs;
-        const uint64_t v = (uint64_t)args;
-        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
-        const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-        return *(const KernelArgs *)(cargs *)(((uint64_t)hi << 32) | lo);
-}
-
-/* The pending DELs of a stepping wavefront's histories, on their records.
- * Out of line: the DEL samplers are the largest code of the path. */
-template <bool F32>
-__device__ __noinline__ void del_wave(
-    const KernelArgs * args, uint32_t slot, bool pending)
-{
-        const KernelArgs & a = uniform_args(args);
-        if (!pending) return;
-        const EngineT<F32> eng = { a.p, a.mv, a.c, a.g, a.ft, a.p, a.rec };
-        Walker w = a.records[slot];
-        eng.walker_del(w);
-        a.records[slot] = w;
-}
-
-/*
- * Stepping: persistent over the step queue of round `parity`. In a round of at
- * most a.wave_del_max histories (or always, a.tail_del > 0) a wavefront
- * applies the DELs of its histories itself instead of queueing them for the
- * next round: the last histories of a batch, and small batches, then run to
- * their end without a round barrier per DEL.
- *
- * The DELs run outside of the stepping loop, on the records: the wavefront
- * saves its histories, calls the DEL code and reloads them, so that nothing
- * of the stepping loop is live in registers across the call. With the call
- * inside the loop the kernel spilled 200 to 1400 registers on every step
- * (12 to 18 without it).
- */
-template <bool F32, bool LDS, bool LEAN, int SCHEME>
-__global__ void __launch_bounds__(512, 2) k_step(KernelArgs args, int parity)
-{
-        KERNEL_ARGS(args);
-        /* With LDS, the tables of the step lookups in the working precision
-         * are read from a copy in LDS: the FP32 mirrors (FP32-bulk), the row
-         * tables (lean FP64 kernels with energy loss) or the packed FP64 step
-         * tables. */
-        using FT = typename std::conditional<LDS && F32, LdsTables,
-            FloatTables>::type;
-        constexpr bool ROWS = LEAN && LDS && !F32 && (SCHEME >= MODE_CSDA);
-        using ST = typename std::conditional<ROWS, LdsRowTables,
-            typename std::conditional<LDS, LdsStepTables,
-                PhysicsView>::type>::type;
-        const FT * ft;
-        const ST * st;
-        if constexpr (LDS && F32)
-                ft = &a.ftl;
-        else
-                ft = &a.ft;
-        if constexpr (ROWS)
-                st = &a.rowl;
-        else if constexpr (LDS)
-                st = &a.stl;
-        else
-                st = &a.p;
-        const EngineT<F32, FT, ST, LEAN, SCHEME> eng = { a.p, a.mv, a.c, a.g,
-                *ft, *st, a.rec, a.records };
-        /* The modes with inelastic DELs. The others have no DEL call, and
-         * spill nothing around it (10^6 muons, CSDA: 205 -> 196 ms, FP32 186
-         * -> 181). */
-        constexpr bool DELS = (SCHEME == SCHEME_ANY) || (SCHEME > MODE_CSDA);
-        const uint64_t below = lanes_below();
-        const uint32_t * in = a.q_step[parity];
-        const unsigned long long n_in = a.counters[C_STEP_N0 + parity];
-        if (n_in == 0) return;
-        if constexpr (LDS) {
-                /* The copy (tens of KB to 160 KB, read from L2 by every
-                 * block of the launch), in 16 B words. */
-                float4 * lds = (float4 *)pg_lds_floats;
-                for (int k = 0; k < a.n_lds_pieces; k++) {
-                        const float4 * src = a.lds_piece[k].src;
-                        float4 * dst = lds + a.lds_piece[k].dst;
-                        for (uint32_t i = threadIdx.x; i < a.lds_piece[k].n4;
-                             i += blockDim.x)
-                                dst[i] = src[i];
-                }
-                __syncthreads();
-        }
-        uint32_t slot = 0;
-        bool exhausted = false;
-        /* A round that fits in the resident lanes: each wavefront takes its
-         * share of the queue once, and the queue has nothing more for it.
-         * (Taken from the shared counter instead, a wavefront learns that
-         * only when it asks again, with a lane freed by its first DEL: with
-         * one history per wavefront every DEL cost a round.) The shares are
-         * spread over all wavefronts, first over the blocks, then over the
-         * wavefronts of a block, unless the caller asked for a number of
-         * lanes. */
-        const bool fits = n_in <= a.resident_lanes;
-        uint32_t waves = gridDim.x * (blockDim.x >> 6);
-        if ((blockDim.x == 512) && (n_in > waves * PACK_LANES) &&
-            (n_in <= waves * 32))
-                waves /= 2;
-        const int lanes = (fits && a.lanes_auto) ?
-            (int)((n_in + waves - 1) / waves) :
-            a.lanes_per_wave;
-        const bool lane_on = (int)(threadIdx.x & 63) < lanes;
-        const bool wave_del = (a.tail_del > 0) ||
-            ((a.tail_del == 0) && (n_in <= a.wave_del_max));
-        /* Lanes below which the histories left are handed over. */
-        const int keep = (wave_del || fits) ? 0 : (lanes * HAND_OVER) / 64;
-        unsigned long long steps_acc = 0;
-        bool held = false; /* the lane has a history, saved in its record */
-        uint64_t del_mask = 0; /* lanes with a DEL to apply here */
-        int del_wait = 0;
-        bool finished = false;
-        do {
-                Walker w;
-                w.phase = PHASE_EMPTY;
-                if (held) w = a.records[slot];
-                for (int it = 0;; it++) {
-                        /* Hand over the histories that left the stepping
-                         * phase. */
-                        const bool done = w.phase == PHASE_DONE;
-                        const bool del = w.phase == PHASE_DEL;
-                        if (done) {
-                                if constexpr (LEAN)
-                                        walker_store(a, slot, w,
-                                            a.records[slot], a.states + slot);
-                                else
-                                        walker_store(a, slot, w, w,
-                                            a.states + slot);
-                                steps_acc += w.t.steps;
-                        }
-                        const bool to_del = DELS && del && !wave_del;
-                        uint64_t dels = DELS ? __ballot(del && wave_del) : 0;
-                        if (dels) {
-                                const int others = __popcll(
-                                    __ballot((w.phase == PHASE_STEP) ||
-                                        (w.phase == PHASE_EHS)));
-                                const int waiting = __popcll(dels);
-                                if ((waiting < others) &&
-                                    (waiting < DEL_BATCH) &&
-                                    (++del_wait <= DEL_WAIT))
-                                        dels = 0; /* not yet */
-                                else
-                                        del_wait = 0;
-                        }
-                        bool to_step = false;
-                        if (keep && exhausted && (it > HAND_OVER_AFTER)) {
-                                const bool left = (w.phase == PHASE_STEP) ||
-                                    (w.phase == PHASE_EHS);
-                                to_step = left &&
-                                    (__popcll(__ballot(left)) < keep);
-                        }
-                        const bool save = to_del || to_step ||
-                            (dels && (w.phase != PHASE_EMPTY) && !done);
-                        if (save)
-                                walker_save<F32, LEAN>(a.records + slot, w);
-                        queue_append(
-                            a.counters + C_DEL_N, a.q_del, to_del, slot);
-                        queue_append(a.counters + C_STEP_N0 + (parity ^ 1),
-                            a.q_step[parity ^ 1], to_step, slot);
-                        if (dels) {
-                                /* DELs in the wavefront, below. */
-                                held = save;
-                                del_mask = dels;
-                                break;
-                        }
-                        if (done || to_del || to_step)
-                                w.phase = PHASE_EMPTY;
-
-                        /* Refill the free lanes from the step queue. */
-                        if (!exhausted) {
-                                const uint64_t free_lanes = __ballot(
-                                    (w.phase == PHASE_EMPTY) && lane_on);
-                                if (free_lanes) {
-                                        const int count = __popcll(free_lanes);
-                                        unsigned long long base = 0;
-                                        if (fits) {
-                                                base = (unsigned long long)
-                                                    lanes *
-                                                    ((threadIdx.x >> 6) *
-                                                            gridDim.x +
-                                                        blockIdx.x);
-                                                exhausted = true;
-                                        } else {
-                                                const int leader =
-                                                    __ffsll((unsigned long
-                                                        long)free_lanes) - 1;
-                                                if ((int)(threadIdx.x & 63) ==
-                                                    leader)
-                                                        base = atomicAdd(
-                                                            a.counters +
-                                                                C_TAKEN,
-                                                            count);
-                                                base = __shfl(
-                                                    base, leader, 64);
-                                                if (base + count >= n_in)
-                                                        exhausted = true;
-                                        }
-                                        if ((w.phase == PHASE_EMPTY) &&
-                                            lane_on) {
-                                                const unsigned long long k =
-                                                    base +
-                                                    __popcll(
-                                                        free_lanes & below);
-                                                if (k < n_in) {
-                                                        slot = in[k];
-                                                        w = a.records[slot];
-                                                }
-                                        }
-                                }
-                        }
-                        if (!__ballot((w.phase == PHASE_STEP) ||
-                                (w.phase == PHASE_EHS))) {
-                                if (exhausted) {
-                                        finished = true;
-                                        break;
-                                }
-                                continue;
-                        }
-                        if constexpr (LEAN) {
-                                /* In scalar registers: the same for every
-                                 * history. */
-                                w.t.rng.k0 = (uint32_t)a.seed;
-                                w.t.rng.k1 = (uint32_t)(a.seed >> 32);
-                                w.t.rng.stream = STREAM_TRANSPORT;
-                                w.slot = slot;
-                        }
-                        if (w.phase == PHASE_STEP) eng.walker_step(w);
-
-                        /* Elastic hard scatterings, on ~16% of the steps of
-                         * a muon in rock, run once enough lanes wait for one
-                         * (half of the lanes in flight, at most a.ehs_batch)
-                         * or none can step, so that the wavefront runs that
-                         * code with most lanes busy. */
-                        const uint64_t ehs = __ballot(w.phase == PHASE_EHS);
-                        const uint64_t stepping =
-                            __ballot(w.phase == PHASE_STEP);
-                        const int waiting = __popcll(ehs);
-                        const int in_flight = waiting + __popcll(stepping);
-                        const int batch =
-                            (in_flight + 1) / 2 < a.ehs_batch ?
-                            (in_flight + 1) / 2 :
-                            a.ehs_batch;
-                        if (ehs && ((waiting >= batch) || !stepping)) {
-                                if (w.phase == PHASE_EHS) eng.walker_ehs(w);
-                        }
-                }
-                if constexpr (DELS) {
-                        if (!finished)
-                                del_wave<F32>(&a, slot,
-                                    (del_mask >> (threadIdx.x & 63)) & 1);
-                }
-        } while (!finished);
-        steps_flush(a, steps_acc);
-}
-
 /* Inelastic DELs of round `parity`, one lane per queued history; the
  * histories go back to the next round's step queue. */
 template <bool F32>
@@ -1515,30 +967,7 @@ struct Launch {
         bool closed; /* every history takes the closed form CSDA */
 };
 
-/* The stepping kernel of a launch. The lean kernels are compiled for one energy
- * loss mode; the general one serves the launches with a frame recorder. In the
- * general kernel, 10^6 muons through the slabs took, without energy loss, 65 ms
- * (FP32 65) instead of 50 (42), and with the tables in HBM, CSDA, 277 ms (288)
- * instead of 216 (193). */
-using StepKernel = void (*)(KernelArgs, int);
-
-template <bool F32, bool LDS>
-StepKernel step_kernel(const KernelArgs & a)
-{
-        if (a.rec.frames != nullptr) return k_step<F32, LDS, false, SCHEME_ANY>;
-        switch (a.c.energy_loss) {
-        case MODE_STRAGGLED:
-                return k_step<F32, LDS, true, MODE_STRAGGLED>;
-        case MODE_MIXED:
-                return k_step<F32, LDS, true, MODE_MIXED>;
-        case MODE_CSDA:
-                return k_step<F32, LDS, true, MODE_CSDA>;
-        default:
-                return k_step<F32, LDS, true, SCHEME_NONE>;
-        }
-}
-
-/* Whether that kernel reads the row tables from its LDS copy. */
+/* Whether the stepping kernel reads the row tables from its LDS copy. */
 bool row_launch(const KernelArgs & a, bool f32)
 {
         return !f32 && (a.rec.frames == nullptr) &&
@@ -1546,17 +975,17 @@ bool row_launch(const KernelArgs & a, bool f32)
             (a.c.energy_loss <= MODE_STRAGGLED);
 }
 
-StepKernel step_kernel(const KernelArgs & a, bool f32, bool lds)
+StepKernel launch_kernel(const KernelArgs & a, bool f32, bool lds)
 {
-        if (f32) return lds ? step_kernel<true, true>(a) :
-                              step_kernel<true, false>(a);
-        return lds ? step_kernel<false, true>(a) : step_kernel<false, false>(a);
+        const bool recorder = a.rec.frames != nullptr;
+        return f32 ? step_kernel<true>(a.c.energy_loss, recorder, lds) :
+                     step_kernel<false>(a.c.energy_loss, recorder, lds);
 }
 
 template <bool F32>
 void launch_step(const KernelArgs & a, int parity, const Launch & L)
 {
-        hipLaunchKernelGGL(step_kernel(a, F32, L.lds_bytes > 0),
+        hipLaunchKernelGGL(launch_kernel(a, F32, L.lds_bytes > 0),
             dim3(L.step_grid), dim3(L.block), L.lds_bytes, L.stream, a, parity);
 }
 
@@ -1615,7 +1044,7 @@ enum pumas_return lds_tables_size(const pumas_gpu_physics * physics,
         }
         if (need > 65536) {
                 const enum pumas_return rc =
-                    allow_lds(step_kernel(a, f32, true), (int)need);
+                    allow_lds(launch_kernel(a, f32, true), (int)need);
                 if (rc != PUMAS_RETURN_SUCCESS) return rc;
         }
         *bytes = (unsigned)need;

@@ -1,0 +1,4 @@
+/* The FP32-bulk stepping kernels. */
+#include "k_step.h"
+
+template StepKernel step_kernel<true>(int, bool, bool);

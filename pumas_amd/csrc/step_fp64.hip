@@ -1,0 +1,4 @@
+/* The FP64 stepping kernels. */
+#include "k_step.h"
+
+template StepKernel step_kernel<false>(int, bool, bool);
