@@ -44,12 +44,15 @@ enum {
         PHASE_DONE
 };
 
+/* Frames recorded of a history: none, of its events, or of its steps too. */
+enum { RECORD_NONE = 0, RECORD_EVENTS, RECORD_STEPS };
+
 /* A history in flight: its Track and the loop carried variables of the
  * reference's stepping loop (src/pumas.c:5231-5273). */
 struct Walker {
         Track t;
         int phase;
-        int record; /* frames of this history are recorded */
+        int record; /* RECORD_...: frames of this history that are recorded */
         int event, rc;
         int media0, end_medium;
         int medium, material, straight, step_index, step_max_type;
@@ -120,12 +123,10 @@ PG_FN bool loop_stalled(Track & t, int & iterations, int limit)
         return true;
 }
 
-/* Appends a frame of `t` to the recorder. Out of line, with its arguments
- * copied: neither the history nor the engine object is pinned to memory on
- * the paths that do not record. */
-static PG_NOINLINE void record_state(const Recorder rec, const Track t,
-    int medium,
-    int event)
+/* Appends a frame of `t`, with the charge and the decay flag of `ct`, to the
+ * recorder. */
+PG_FN void record_append(const Recorder & rec, const Track & t,
+    const Track & ct, int medium, int event)
 {
 #ifdef __HIP_DEVICE_COMPILE__
         const unsigned long long k = atomicAdd(rec.count, 1ull);
@@ -134,7 +135,7 @@ static PG_NOINLINE void record_state(const Recorder rec, const Track t,
 #endif
         if (k >= rec.capacity) return;
         Frame & f = rec.frames[k];
-        f.charge = t.charge;
+        f.charge = ct.charge;
         f.energy = t.energy;
         f.distance = t.distance;
         f.grammage = t.grammage;
@@ -144,12 +145,20 @@ static PG_NOINLINE void record_state(const Recorder rec, const Track t,
                 f.position[j] = t.pos[j];
                 f.direction[j] = t.dir[j];
         }
-        f.decayed = t.decayed;
+        f.decayed = ct.decayed;
         f.medium = medium;
         f.event = event;
         f.pad = 0;
         f.history = ((uint64_t)t.rng.h1 << 32) | t.rng.h0;
         f.reserved = 0;
+}
+
+/* The same out of line, with its arguments copied: neither the history nor the
+ * engine object is pinned to memory on the paths that do not record. */
+static PG_NOINLINE void record_state(const Recorder rec, const Track t,
+    int medium, int event)
+{
+        record_append(rec, t, t, medium, event);
 }
 
 /* SCHEME of an engine that reads the energy loss mode from its Config: any
@@ -166,7 +175,7 @@ constexpr int SCHEME_NONE = -3;
  * geometry stay in double precision.
  */
 template <bool F32, class FT = FloatTables, class ST = PhysicsView,
-    bool LEAN = false, int SCHEME = SCHEME_ANY>
+    bool LEAN = false, int SCHEME = SCHEME_ANY, bool RECORD = true>
 struct EngineT {
         const PhysicsView & p;
         const ModelView & mv;
@@ -183,8 +192,7 @@ struct EngineT {
         /* The members of a Walker that only its events and its end touch
          * (ids and end conditions, the limits of the other energy loss
          * modes): a lean engine, which keeps the rest of the Walker in
-         * registers over many steps, leaves them in the record. A lean
-         * engine does not record frames. */
+         * registers over many steps, leaves them in the record. */
         PG_FN Walker & cold(Walker & w) const
         {
                 if constexpr (LEAN)
@@ -193,14 +201,24 @@ struct EngineT {
                         return w;
         }
 
+        /* Whether frames of the history, or of its steps, are recorded (RECORD
+         * false: in a launch without a recorder). */
+        PG_FN bool recorded(const Walker & w, int which = RECORD_EVENTS) const
+        {
+                return RECORD && (w.record >= which);
+        }
+
         /* Records the state of `w` in `medium` with `event`, if the history
-         * is recorded (record_state, src/pumas.c:7738-7780). */
+         * is recorded (record_state, src/pumas.c:7738-7780). In line in a
+         * lean engine: a call in the stepping loop spills registers. */
         PG_FN void record_frame(const Walker & w, int medium, int event) const
         {
-                if constexpr (!LEAN) {
-                        if (!w.record) return;
+                if (!recorded(w)) return;
+                if constexpr (LEAN)
+                        record_append(
+                            rec, w.t, records[w.slot].t, medium, event);
+                else
                         record_state(rec, w.t, medium, event);
-                }
         }
 
         /* The energy loss mode (a constant when the engine is compiled for
@@ -1995,8 +2013,11 @@ struct EngineT {
                 {
                         const uint64_t id =
                             ((uint64_t)t.rng.h1 << 32) | t.rng.h0;
-                        w.record = (rec.frames != nullptr) &&
+                        const bool record = (rec.frames != nullptr) &&
                             (id >= rec.first) && (id < rec.last);
+                        w.record = !record ? RECORD_NONE :
+                            (rec.period > 0)  ? RECORD_STEPS :
+                                                RECORD_EVENTS;
                 }
                 if (t.decayed) {
                         w.event = EVENT_VERTEX_DECAY;
@@ -2168,8 +2189,12 @@ struct EngineT {
                 const int scheme = loss();
                 w.ti = t.time;
                 /* A lean engine's weight changes at events only, each of
-                 * which ends here: its initial weight is the weight. */
-                if constexpr (!LEAN) w.wi = t.weight;
+                 * which ends here, and at recorded steps: without those its
+                 * initial weight is the weight. */
+                if (!LEAN)
+                        w.wi = t.weight;
+                else if (recorded(w, RECORD_STEPS))
+                        cold(w).wi = t.weight;
                 /* The grammage is read by the limits of the CSDA and mixed
                  * modes only, the energy loss by the backward weights. */
                 const double Xi = t.grammage;
@@ -2233,20 +2258,22 @@ struct EngineT {
                 w.step_index++;
                 /* Recorded steps, src/pumas.c:5296-5328: every period-th
                  * step also gets the event-time weight update. */
-                const int record_step = !LEAN && w.record && (rec.period > 0) &&
+                const bool record_steps = recorded(w, RECORD_STEPS);
+                const bool record_step = record_steps &&
                     (w.step_index != 1) && ((w.step_index % rec.period) == 0);
                 if (!t.step_event && !record_step) return;
+                const double wi =
+                    (LEAN && !record_steps) ? t.weight : cold(w).wi;
 
                 if ((c.direction == MODE_BACKWARD) &&
                     (loss() >= MODE_CSDA)) {
                         const double wt = (c.decay == MODE_WEIGHTED) ?
                             lm::exp(-fabs(t.time - w.ti) / p.ctau) :
                             1.;
-                        t.weight = (LEAN ? t.weight : w.wi) * wt * w.dei *
+                        t.weight = wi * wt * w.dei *
                             event_energy_loss(t, scheme, w.material);
                 } else if (c.decay == MODE_WEIGHTED) {
-                        t.weight = (LEAN ? t.weight : w.wi) *
-                            lm::exp(-fabs(t.time - w.ti) / p.ctau);
+                        t.weight = wi * lm::exp(-fabs(t.time - w.ti) / p.ctau);
                 }
 
                 if (!t.step_event) {
@@ -2316,7 +2343,7 @@ struct EngineT {
                 /* Pre and post DEL points when recording, src/pumas.c:
                  * 5343-5387: the pre point is the state after the DEL with
                  * its energy and direction before it. */
-                const int rec_del = !LEAN && w.record && (rec.period > 0);
+                const bool rec_del = recorded(w, RECORD_STEPS);
                 const double ki = t.energy;
                 const double ui[3] = { t.dir[0], t.dir[1], t.dir[2] };
                 {

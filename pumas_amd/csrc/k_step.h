@@ -49,17 +49,17 @@ __device__ __noinline__ void del_wave(
  * inside the loop the kernel spilled 200 to 1400 registers on every step
  * (12 to 18 without it).
  */
-template <bool F32, bool LDS, bool LEAN, int SCHEME>
+template <bool F32, bool LDS, bool RECORD, int SCHEME>
 __global__ void __launch_bounds__(512, 2) k_step(KernelArgs args, int parity)
 {
         KERNEL_ARGS(args);
         /* With LDS, the tables of the step lookups in the working precision
          * are read from a copy in LDS: the FP32 mirrors (FP32-bulk), the row
-         * tables (lean FP64 kernels with energy loss) or the packed FP64 step
+         * tables (FP64 with energy loss) or the packed FP64 step
          * tables. */
         using FT = typename std::conditional<LDS && F32, LdsTables,
             FloatTables>::type;
-        constexpr bool ROWS = LEAN && LDS && !F32 && (SCHEME >= MODE_CSDA);
+        constexpr bool ROWS = LDS && !F32 && (SCHEME >= MODE_CSDA);
         using ST = typename std::conditional<ROWS, LdsRowTables,
             typename std::conditional<LDS, LdsStepTables,
                 PhysicsView>::type>::type;
@@ -75,12 +75,12 @@ __global__ void __launch_bounds__(512, 2) k_step(KernelArgs args, int parity)
                 st = &a.stl;
         else
                 st = &a.p;
-        const EngineT<F32, FT, ST, LEAN, SCHEME> eng = { a.p, a.mv, a.c, a.g,
-                *ft, *st, a.rec, a.records };
+        const EngineT<F32, FT, ST, true, SCHEME, RECORD> eng = { a.p, a.mv, a.c,
+                a.g, *ft, *st, a.rec, a.records };
         /* The modes with inelastic DELs. The others have no DEL call, and
          * spill nothing around it (10^6 muons, CSDA: 205 -> 196 ms, FP32 186
          * -> 181). */
-        constexpr bool DELS = (SCHEME == SCHEME_ANY) || (SCHEME > MODE_CSDA);
+        constexpr bool DELS = SCHEME > MODE_CSDA;
         const uint64_t below = lanes_below();
         const uint32_t * in = a.q_step[parity];
         const unsigned long long n_in = a.counters[C_STEP_N0 + parity];
@@ -136,12 +136,8 @@ __global__ void __launch_bounds__(512, 2) k_step(KernelArgs args, int parity)
                         const bool done = w.phase == PHASE_DONE;
                         const bool del = w.phase == PHASE_DEL;
                         if (done) {
-                                if constexpr (LEAN)
-                                        walker_store(a, slot, w,
-                                            a.records[slot], a.states + slot);
-                                else
-                                        walker_store(a, slot, w, w,
-                                            a.states + slot);
+                                walker_store(a, slot, w, a.records[slot],
+                                    a.states + slot);
                                 steps_acc += w.t.steps;
                         }
                         const bool to_del = DELS && del && !wave_del;
@@ -168,7 +164,7 @@ __global__ void __launch_bounds__(512, 2) k_step(KernelArgs args, int parity)
                         const bool save = to_del || to_step ||
                             (dels && (w.phase != PHASE_EMPTY) && !done);
                         if (save)
-                                walker_save<F32, LEAN>(a.records + slot, w);
+                                walker_save<F32>(a.records + slot, w);
                         queue_append(
                             a.counters + C_DEL_N, a.q_del, to_del, slot);
                         queue_append(a.counters + C_STEP_N0 + (parity ^ 1),
@@ -232,14 +228,11 @@ __global__ void __launch_bounds__(512, 2) k_step(KernelArgs args, int parity)
                                 }
                                 continue;
                         }
-                        if constexpr (LEAN) {
-                                /* In scalar registers: the same for every
-                                 * history. */
-                                w.t.rng.k0 = (uint32_t)a.seed;
-                                w.t.rng.k1 = (uint32_t)(a.seed >> 32);
-                                w.t.rng.stream = STREAM_TRANSPORT;
-                                w.slot = slot;
-                        }
+                        /* In scalar registers: the same for every history. */
+                        w.t.rng.k0 = (uint32_t)a.seed;
+                        w.t.rng.k1 = (uint32_t)(a.seed >> 32);
+                        w.t.rng.stream = STREAM_TRANSPORT;
+                        w.slot = slot;
                         if (w.phase == PHASE_STEP) eng.walker_step(w);
 
                         /* Elastic hard scatterings, on ~16% of the steps of
@@ -269,32 +262,32 @@ __global__ void __launch_bounds__(512, 2) k_step(KernelArgs args, int parity)
         steps_flush(a, steps_acc);
 }
 
-/* The stepping kernel of a launch. The lean kernels are compiled for one energy
- * loss mode; the general one serves the launches with a frame recorder. In the
- * general kernel, 10^6 muons through the slabs took, without energy loss, 65 ms
- * (FP32 65) instead of 50 (42), and with the tables in HBM, CSDA, 277 ms (288)
- * instead of 216 (193). */
-template <bool F32, bool LDS>
-StepKernel step_kernel_mode(int energy_loss, bool recorder)
+/* The stepping kernel of a launch: compiled for its energy loss mode, and with
+ * or without a frame recorder. In one kernel for every mode, which launches with
+ * a recorder, with the tables in HBM or without energy loss took, 10^6 muons
+ * through the slabs: recorder, CSDA 252 ms (FP32 247) instead of 199 (186), no
+ * loss 66 (65) instead of 51 (44); HBM, CSDA 277 (288) instead of 216 (193). With
+ * the recorder's code in all of them, launches without one lose 1 to 6 %. */
+template <bool F32, bool LDS, bool RECORD>
+StepKernel step_kernel_mode(int energy_loss)
 {
-        if (recorder) return k_step<F32, LDS, false, SCHEME_ANY>;
         switch (energy_loss) {
         case MODE_STRAGGLED:
-                return k_step<F32, LDS, true, MODE_STRAGGLED>;
+                return k_step<F32, LDS, RECORD, MODE_STRAGGLED>;
         case MODE_MIXED:
-                return k_step<F32, LDS, true, MODE_MIXED>;
+                return k_step<F32, LDS, RECORD, MODE_MIXED>;
         case MODE_CSDA:
-                return k_step<F32, LDS, true, MODE_CSDA>;
+                return k_step<F32, LDS, RECORD, MODE_CSDA>;
         default:
-                return k_step<F32, LDS, true, SCHEME_NONE>;
+                return k_step<F32, LDS, RECORD, SCHEME_NONE>;
         }
 }
 
-template <bool F32>
-StepKernel step_kernel(int energy_loss, bool recorder, bool lds)
+template <bool F32, bool RECORD>
+StepKernel step_kernel(int energy_loss, bool lds)
 {
-        return lds ? step_kernel_mode<F32, true>(energy_loss, recorder) :
-                     step_kernel_mode<F32, false>(energy_loss, recorder);
+        return lds ? step_kernel_mode<F32, true, RECORD>(energy_loss) :
+                     step_kernel_mode<F32, false, RECORD>(energy_loss);
 }
 
 #endif

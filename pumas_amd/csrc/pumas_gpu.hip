@@ -970,16 +970,18 @@ struct Launch {
 /* Whether the stepping kernel reads the row tables from its LDS copy. */
 bool row_launch(const KernelArgs & a, bool f32)
 {
-        return !f32 && (a.rec.frames == nullptr) &&
-            (a.c.energy_loss >= MODE_CSDA) &&
+        return !f32 && (a.c.energy_loss >= MODE_CSDA) &&
             (a.c.energy_loss <= MODE_STRAGGLED);
 }
 
 StepKernel launch_kernel(const KernelArgs & a, bool f32, bool lds)
 {
-        const bool recorder = a.rec.frames != nullptr;
-        return f32 ? step_kernel<true>(a.c.energy_loss, recorder, lds) :
-                     step_kernel<false>(a.c.energy_loss, recorder, lds);
+        const int loss = a.c.energy_loss;
+        if (a.rec.frames != nullptr)
+                return f32 ? step_kernel<true, true>(loss, lds) :
+                             step_kernel<false, true>(loss, lds);
+        return f32 ? step_kernel<true, false>(loss, lds) :
+                     step_kernel<false, false>(loss, lds);
 }
 
 template <bool F32>

@@ -194,15 +194,11 @@ __device__ __forceinline__ void walker_store(const KernelArgs & a, uint64_t i,
                 atomicCAS(a.counters + C_ERROR, 0ull, (unsigned long long)rc);
 }
 
-/* Write a history back to its record; of a lean engine, only the members
- * that it keeps in registers. */
-template <bool F32, bool LEAN>
+/* Write a history of a lean engine back to its record: the members that it
+ * keeps in registers. */
+template <bool F32>
 __device__ __forceinline__ void walker_save(Walker * r, const Walker & w)
 {
-        if constexpr (!LEAN) {
-                *r = w;
-                return;
-        }
         r->t.energy = w.t.energy;
         r->t.distance = w.t.distance;
         r->t.grammage = w.t.grammage;
@@ -299,11 +295,12 @@ constexpr int HAND_OVER = 40;
 constexpr int HAND_OVER_AFTER = 32;
 constexpr uint32_t PACK_LANES = 8;
 
-/* The stepping kernel of a launch, in an energy loss mode (step_fp64.hip,
- * step_fp32.hip: compiled apart, which is most of the build's time). */
+/* The stepping kernel of a launch, in an energy loss mode, with the tables in
+ * LDS or in HBM (step_*.hip: compiled apart, which is most of the build's
+ * time). */
 using StepKernel = void (*)(KernelArgs, int);
 
-template <bool F32>
-StepKernel step_kernel(int energy_loss, bool recorder, bool lds);
+template <bool F32, bool RECORD>
+StepKernel step_kernel(int energy_loss, bool lds);
 
 #endif

@@ -1,4 +1,4 @@
 /* The FP32-bulk stepping kernels. */
 #include "k_step.h"
 
-template StepKernel step_kernel<true>(int, bool, bool);
+template StepKernel step_kernel<true, false>(int, bool);

@@ -1,4 +1,4 @@
 /* The FP64 stepping kernels. */
 #include "k_step.h"
 
-template StepKernel step_kernel<false>(int, bool, bool);
+template StepKernel step_kernel<false, false>(int, bool);

@@ -2,12 +2,18 @@
 read from HBM instead of LDS, no energy loss, and a frame recorder. Times are
 the best of five calls of 10^6 muons through the slab stack, in turn; results
 are equal (test_gpu_parity, test_gpu_fp32, test_gpu_recorder)."""
+import ctypes
 import time
 
 import numpy as np
 import pytest
 
+from parity import assert_parity
+from test_gpu_recorder import grouped
+from test_host_engine import build_host, run_host
+
 import pumas_amd as pa
+from pumas_amd import _abi
 from pumas_amd import workloads as W
 
 pytestmark = pytest.mark.gpu
@@ -56,3 +62,69 @@ def test_no_energy_loss(gpu_standard, precision):
     a, b = step_times(gpu_standard, [(csda, dict(precision=precision)),
                                      (none, dict(precision=precision))])
     assert b < 1.05 * a
+
+
+@pytest.mark.parametrize("precision", PRECISIONS)
+@pytest.mark.parametrize("loss", [pa.Mode.CSDA, pa.Mode.DISABLED])
+def test_recorder(gpu_standard, loss, precision):
+    """A recorder of a hundred of the 10^6 histories."""
+    ctx = W.slabs_forward_context(energy_loss=loss).replace(
+        event=pa.Event.LIMIT_DISTANCE, limit_distance=500.0)
+    rec = pa.Recorder(1 << 16, period=0, first_history=0, n_histories=100)
+    plain, recorded = step_times(gpu_standard, [
+        (ctx, dict(precision=precision)),
+        (ctx, dict(precision=precision, recorder=rec))])
+    assert rec.frames()[1] > 0
+    assert recorded < 1.1 * plain
+
+
+@pytest.mark.parametrize("options", [{}, dict(tail_del=-1),
+                                     dict(lds_tables=-1),
+                                     dict(max_steps=150)], ids=str)
+@pytest.mark.parametrize("period", [0, 1, 7])
+@pytest.mark.parametrize("forward", [True, False])
+@pytest.mark.parametrize("loss", [pa.Mode.DISABLED, pa.Mode.CSDA,
+                                  pa.Mode.MIXED, pa.Mode.STRAGGLED])
+def test_frames_equal_host(gpu_standard, loss, forward, period, options):
+    """Frames and final states of a batch whose middle half is recorded are
+    those of the engine on the host, which steps a history at a time: steps,
+    DELs, medium changes, and histories that a step limit ends."""
+    make = W.slabs_forward_states if forward else W.slabs_backward_states
+    ctx = (W.slabs_forward_context if forward else
+           W.slabs_backward_context)(energy_loss=loss).replace(
+        event=pa.Event.LIMIT_DISTANCE, limit_distance=600.0)
+    desc = W.slabs_geometry()
+    n, first, count, cap = 48, 12, 24, 1 << 20
+    s = make(n, seed=31, **({} if forward else dict(kmax=50.0)))
+    host = build_host()
+    frames, k = np.zeros(cap, _abi.FRAME_DTYPE), ctypes.c_ulonglong(0)
+    host.host_record(frames.ctypes.data, ctypes.addressof(k), cap, period,
+                     first, count)
+    host.host_set_max_steps(options.get("max_steps", 10000000))
+    try:
+        out = run_host(host, "standard_c005", ctx, desc, s, seed=6)
+    finally:
+        host.host_record(None, None, 0, 0, 0, 0)
+        host.host_set_max_steps(10000000)
+    ref = grouped(frames[:k.value])
+    rec = pa.Recorder(cap, period=period, first_history=first,
+                      n_histories=count)
+    gpu = pa.transport(gpu_standard, ctx, pa.Geometry(gpu_standard, desc),
+                       s.copy(), seed=6, recorder=rec, raise_errors=False,
+                       **options)
+    assert_parity(gpu, dict(zip(("final", "events", "media", "steps", "draws",
+                                 "rc"), out)), 1e-12)
+    f, total = rec.frames()
+    assert total == len(ref) and 2 * count <= total <= cap
+    f = grouped(f)
+    for field in ("history", "event", "medium"):
+        np.testing.assert_array_equal(f[field], ref[field])
+    np.testing.assert_array_equal(f["state"]["charge"], ref["state"]["charge"])
+    np.testing.assert_array_equal(f["state"]["decayed"],
+                                  ref["state"]["decayed"])
+    for field in ("energy", "distance", "grammage", "time", "weight"):
+        np.testing.assert_allclose(f["state"][field], ref["state"][field],
+                                   rtol=1e-12, atol=1e-300)
+    for field in ("position", "direction"):
+        np.testing.assert_allclose(f["state"][field], ref["state"][field],
+                                   rtol=0, atol=1e-9)
