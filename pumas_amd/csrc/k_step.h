@@ -110,9 +110,11 @@ __global__ void __launch_bounds__(512, 2) k_step(KernelArgs args, int parity)
          * lanes. */
         const bool fits = n_in <= a.resident_lanes;
         uint32_t waves = gridDim.x * (blockDim.x >> 6);
-        if ((blockDim.x == 512) && (n_in > waves * PACK_LANES) &&
-            (n_in <= waves * 32) &&
-            ((a.g.kind == GEO_INFINITE) || (a.g.kind == GEO_SLABS)))
+        const bool grid =
+            (a.g.kind == GEO_TERRAIN) || (a.g.kind == GEO_VOXELS);
+        if ((blockDim.x == 512) &&
+            (n_in > waves * (grid ? PACK_LANES_GRID : PACK_LANES)) &&
+            (n_in <= waves * 32))
                 waves /= 2;
         const int lanes = (fits && a.lanes_auto) ?
             (int)((n_in + waves - 1) / waves) :

@@ -285,13 +285,14 @@ __device__ __forceinline__ void steps_flush(
  * progress.
  * PACK_LANES: a round that fits with more than so many lanes per wavefront, and
  * in half of the wavefronts of each 512 lane block, is put in that half: one
- * wavefront per SIMD with twice the lanes. 30011 muons 48.2 -> 45.2 ms, 60000
- * 53.4 -> 48.6; below it loses: 3000 29.8 -> 32.7, 10000 38.6 -> 40.6. Not in
- * terrains and voxel grids, whose locations load per lane: 24000 histories, mixed
- * losses, terrain 43.4 -> 48.7 ms, voxels 22.3 -> 25.2, straggled 37.8 -> 40.5 and
- * 19.0 -> 20.9; only near 64000 FP64 ones it gains there (46.9 -> 44.6, 25.5 ->
- * 24.8). Infinite media and slabs gain in every mode: 17000 to 64000 histories
- * 2 to 22 %.
+ * wavefront per SIMD with twice the lanes. In infinite media and slabs: 30011
+ * muons 48.2 -> 45.2 ms, 60000 53.4 -> 48.6, 17000 to 64000 histories 2 to 22 %
+ * in every energy loss mode and precision; below it loses: 3000 29.8 -> 32.7,
+ * 10000 38.6 -> 40.6. In terrains and voxel grids (PACK_LANES_GRID), whose
+ * locations load per lane, it loses longer: 24000 histories, mixed losses,
+ * terrain 43.4 -> 48.7 ms, voxels 22.3 -> 25.2, straggled 37.8 -> 40.5 and 19.0
+ * -> 20.9, 40000 43.0 -> 43.9 and 22.5 -> 23.1; 50021 voxel histories 24.7 ->
+ * 24.1, 64000 46.9 -> 44.6 and 25.5 -> 24.8.
  */
 constexpr uint64_t WAVE_DEL_ROUNDS = 4;
 constexpr int DEL_BATCH = 24;
@@ -299,6 +300,7 @@ constexpr int DEL_WAIT = 48;
 constexpr int HAND_OVER = 40;
 constexpr int HAND_OVER_AFTER = 32;
 constexpr uint32_t PACK_LANES = 8;
+constexpr uint32_t PACK_LANES_GRID = 22;
 
 /* The stepping kernel of a launch, in an energy loss mode, with the tables in
  * LDS or in HBM (step_*.hip: compiled apart, which is most of the build's
