@@ -317,7 +317,9 @@ struct pumas_gpu_options {
         /* Histories per wavefront of the stepping kernel (1 to 64). 0: a
          * batch that does not fill the resident wavefronts is spread over
          * all of them with fewer histories each (lower latency for small
-         * requests); 64: full wavefronts on as few CUs as the batch fills.
+         * requests), and occupies one CU per history up to the whole device;
+         * 64: full wavefronts on as few CUs as the batch fills, for callers
+         * that overlap small calls on several streams (as the server does).
          * Results do not depend on it. */
         int lanes_per_wave;
         /* Iterations after which a rejection or bisection loop gives up

@@ -1,6 +1,7 @@
 /*
- * libpumas_hip: C ABI, table upload, geometry upload and the transport
- * kernels for gfx950 (a wavefront scheduler over per-phase queues, below).
+ * libpumas_hip: C ABI, table upload, geometry upload and the transport for
+ * gfx950: the wavefront scheduler (scheduler.h), its kernels but the stepping
+ * one (k_step.h), and their launches.
  */
 #include <hip/hip_runtime.h>
 
@@ -1014,10 +1015,10 @@ enum pumas_return allow_lds(StepKernel kernel, int bytes)
         return PUMAS_RETURN_SUCCESS;
 }
 
-/* Bytes of the LDS copy of the step tables in the stepping kernel, or 0
- * when `per_cu` copies do not fit in the LDS of a CU; sets the pieces of the
- * copy. Row tables are smaller than the step tables (they hold one energy
- * loss scheme), which decide. */
+/* Bytes of the LDS copy of the tables in the stepping kernel, or 0 when the
+ * step tables (the FP32 mirrors in FP32-bulk) do not fit `per_cu` times in the
+ * LDS of a CU; sets the pieces of the copy. FP64 launches with energy loss copy
+ * the row tables instead, which are smaller: they hold one energy loss scheme. */
 enum pumas_return lds_tables_size(const pumas_gpu_physics * physics,
     KernelArgs & a, int device, int per_cu, bool f32, unsigned * bytes)
 {
@@ -1082,14 +1083,14 @@ enum pumas_return transport_chunk(const KernelArgs & a0, size_t base,
     unsigned long long * error, struct pumas_gpu_stats * stats,
     void * fixed = nullptr)
 {
-        /* No more resident blocks than the chunk fills with histories, so
-         * that a small request takes full wavefronts on few CUs and leaves
-         * the rest of the device to concurrent requests. */
+        /* No more resident blocks than the chunk fills with histories: with a
+         * given number of lanes per wavefront, a small request leaves the rest
+         * of the device to concurrent requests. */
         const size_t resident = (size_t)L.n_cu * L.per_cu;
         const size_t waves = (size_t)(L.block / 64);
         /* Spread (0): as many blocks as histories, up to all the resident
-         * ones; a round that fits in them shares its histories out over
-         * every wavefront (k_step). */
+         * ones, each of which takes a CU; a round that fits in them shares its
+         * histories out over their wavefronts (k_step). */
         const bool lanes_auto = L.lanes_per_wave <= 0;
         const int lanes = lanes_auto ? 64 : L.lanes_per_wave;
         const size_t per_block = lanes_auto ? 1 : waves * (size_t)lanes;
